@@ -1352,7 +1352,7 @@ vkv_status matmul_impl(const float *x, int32_t n_cols, int64_t n_in, const float
     a.norm_w = norm_w;
     a.norm_b = norm_b;
     a.ada = ada;
-    if (!in_place && gemm_fused_ok(a, n_col_tiles)) {
+    if (!in_place && gemm_fused_ok(a)) {
         a.x = x;
         a.x_stride = n_in;
         a.x_ring = in_rows.ring;

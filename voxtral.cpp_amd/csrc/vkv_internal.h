@@ -195,6 +195,9 @@ struct MmArgs {
     float rope_ts;
     int32_t rope_hd;
     int64_t rope_pos0;
+    // k_gemm_wide: the waves that k_gemm_kq splits K over for these matrices
+    // (set by launch_gemm_kq)
+    int32_t kw;
     MmOut out[kMvMaxOuts];
 };
 
@@ -207,11 +210,9 @@ hipError_t launch_q8k_rows(const float *x, int64_t x_stride, int x_ring, int x_r
                            float eps, int8_t *codes, float *xd, int16_t *bs16, bool q80,
                            hipStream_t st);
 hipError_t launch_gemm_kq(MmArgs a, int n_col_tiles, hipStream_t st);
-// input rows one work group of launch_gemm_kq covers for this call
-int gemm_cols_per_wg(const MmArgs &a, int n_col_tiles);
 // whether launch_gemm_kq may quantize this call's input inside its work
 // groups (MmArgs::x): few (row, block) tasks per work group, LDS to spare
-bool gemm_fused_ok(const MmArgs &a, int n_col_tiles);
+bool gemm_fused_ok(const MmArgs &a);
 hipError_t launch_q8k_quant(const float *x, int n, const float *norm_w, const float *ada, float eps,
                             uint8_t *out, hipStream_t st);
 hipError_t launch_kq_dequant(int dtype, const uint8_t *src, int64_t n, const float *add, float *y,

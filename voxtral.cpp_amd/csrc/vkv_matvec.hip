@@ -1449,6 +1449,19 @@ __device__ __forceinline__ void gemm_hdr(const GFragQ8 &f, uint32_t (*hdr)[6], i
     }
 }
 
+// A 256-block's share of an output from its exact integer sums, as explicit
+// fma's: every multi-row kernel adds a block by the same operations, so an
+// output's bits do not depend on which kernel its call's size selects.
+__device__ __forceinline__ float q4_block_term(float dw, float dmw, float dx, float isum, float imin,
+                                               float acc) {
+#pragma clang fp contract(off)
+    return acc + fmaf(dx * dw, isum, -((dx * dmw) * imin));
+}
+__device__ __forceinline__ float q6_block_term(float dw, float dx, float isum, float acc) {
+#pragma clang fp contract(off)
+    return fmaf(dx * dw, isum, acc);
+}
+
 // Q8_0: block j's exact integer sums, times fp16(d_w) * fp16(d_x) (ggml's
 // per-block term of vec_dot_q8_0_q8_0)
 __device__ __forceinline__ void gemm_dot(const GFragQ8 &f, const GFragX &x, const uint32_t (&hd)[4][5],
@@ -1485,10 +1498,9 @@ __device__ __forceinline__ void gemm_dot(const GFragQ4 &f, const GFragX &x, cons
         }
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float d = h2f(hd[i][0] & 0xffffu) * x.dx, dmin = h2f(hd[i][0] >> 16) * x.dx;
-        acc[i] += d * (float)isum[i] - dmin * (float)imin[i];
-    }
+    for (int i = 0; i < 4; ++i)
+        acc[i] = q4_block_term(h2f(hd[i][0] & 0xffffu), h2f(hd[i][0] >> 16), x.dx, (float)isum[i],
+                               (float)imin[i], acc[i]);
 }
 
 __device__ __forceinline__ void gemm_dot(const GFragQ6 &f, const GFragX &x, const uint32_t (&hd)[4][5],
@@ -1516,7 +1528,8 @@ __device__ __forceinline__ void gemm_dot(const GFragQ6 &f, const GFragX &x, cons
             }
         }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] += (h2f(hd[i][0]) * x.dx) * (float)isum[i];
+    for (int i = 0; i < 4; ++i)
+        acc[i] = q6_block_term(h2f(hd[i][0]), x.dx, (float)isum[i], acc[i]);
 }
 
 // RoPE (ggml mode 0) of one element of a pair in the products' epilogue,
@@ -1529,6 +1542,17 @@ __device__ __forceinline__ float rope_elem(float self, float partner, bool odd, 
     for (int i = 0; i < pair; ++i) theta *= ts;
     const float c = (float)cos((double)theta), sn = (float)sin((double)theta);
     return odd ? partner * sn + self * c : self * c - partner * sn;
+}
+
+// Both elements of a pair at once (one angle): the same bits as rope_elem's
+__device__ __forceinline__ void rope_pair(float &even, float &odd, int pair, float pos, float ts) {
+#pragma clang fp contract(off)
+    float theta = pos;
+    for (int i = 0; i < pair; ++i) theta *= ts;
+    const float c = (float)cos((double)theta), sn = (float)sin((double)theta);
+    const float e = even, o = odd;
+    even = e * c - o * sn;
+    odd = e * sn + o * c;
 }
 
 // Waves per work group: 8, or 16 when a call has few 16-row tiles (the
@@ -1739,6 +1763,477 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))
     else run(std::integral_constant<int, kWQ6>{});
 }
 
+// ---------------------------------------------------------------------------
+// The same products for many input rows.  k_gemm_kq gives each 16-row tile its
+// own work group, which reads the whole input image again; from about
+// kWideCols input rows that re-reading from L2 is what it spends its time on.
+// Here a work group owns 64 weight rows x 16 CT input rows: wave w rows
+// [16 w, 16 w + 16), every wave the same input columns, whose image block is
+// staged in LDS once per K block (double-buffered, one barrier per block; the
+// next block's weights and image are requested before the current one's
+// products).
+//
+// Products per 256-block.  The 6-bit scales are folded into the int8 operand
+// instead of multiplying each 32-element sum on the VALU, which took ~70 of
+// the ~90 VALU operations per tile and block: a Q4_K code times 3 bits of its
+// scale fits int8 (15 x 7), so with sc = 8 h + l the block's sum is
+// 8 sum (q h) x + sum (q l) x, two chains of four v_mfma_i32_16x16x64_i8; a
+// Q6_K code (-32 .. 31) times a digit of -3 .. 3 does too, and an int8 scale
+// is 49 a + 7 b + c with such digits: three chains.  The mins' sum is one
+// v_mfma_f32_16x16x16_f16: mins (and 64 mins) against the 32-element sums
+// split into 6 low bits and the rest, all integers that f16 holds, summed
+// below 2^24.  Every sum is the exact integer, and the blocks are added in
+// k_gemm_kq's order (virtual wave v of a.kw: blocks v, v + kw, ..; then the
+// waves in order), so both kernels give the same bits.  Q8_0 blocks have a
+// float scale per 32 elements: one v_mfma_i32_16x16x32_i8 each.
+// ---------------------------------------------------------------------------
+typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 h4_t __attribute__((ext_vector_type(4)));
+typedef float f4_t __attribute__((ext_vector_type(4)));
+
+// a 16- or 8-byte load at an even address
+struct __attribute__((packed, aligned(2))) Even16 {
+    uint32_t w[4];
+};
+struct __attribute__((packed, aligned(2))) Even8 {
+    uint32_t w[2];
+};
+struct __attribute__((packed, aligned(4))) Dword16 {
+    uint32_t w[4];
+};
+__device__ __forceinline__ u32x4_t ld16(const uint8_t *p) {
+    const Dword16 v = *reinterpret_cast<const Dword16 *>(p);
+    return u32x4_t{v.w[0], v.w[1], v.w[2], v.w[3]};
+}
+__device__ __forceinline__ u32x4_t ld16_even(const uint8_t *p) {
+    const Even16 v = *reinterpret_cast<const Even16 *>(p);
+    return u32x4_t{v.w[0], v.w[1], v.w[2], v.w[3]};
+}
+
+__device__ __forceinline__ uint32_t pk_mul(uint32_t a, uint32_t b) {
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2_t, a) * __builtin_bit_cast(u16x2_t, b));
+}
+__device__ __forceinline__ uint32_t pk_mad(uint32_t a, uint32_t b, uint32_t c) {
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2_t, a) * __builtin_bit_cast(u16x2_t, b) +
+                                            __builtin_bit_cast(u16x2_t, c));
+}
+
+// A lane's raw bytes of one block of its weight row (row lane & 15 of the
+// wave's tile, kg = lane >> 4).
+template <int WK>
+struct WideRaw;
+template <>
+struct WideRaw<kWQ4> {
+    u32x4_t h;      // header: d | dmin, scales and mins
+    u32x4_t q[2];   // code bytes 16 u .. +15, u = kg, kg + 4
+    __device__ __forceinline__ void load(const uint8_t *blk, int kg) {
+        h = ld16(blk);
+        q[0] = ld16(blk + 16 + 16 * kg);
+        q[1] = ld16(blk + 80 + 16 * kg);
+    }
+};
+template <>
+struct WideRaw<kWQ6> {
+    u32x4_t l0, l1, hi;   // ql (g even), ql (g odd), qh of elements 16 (kg & 1) .. of half kg >> 1
+    Even8 sc;             // the half's 8 scales
+    uint32_t d;
+    __device__ __forceinline__ void load(const uint8_t *blk, int kg) {
+        const int n = kg >> 1, e = 16 * (kg & 1);
+        l0 = ld16_even(blk + 64 * n + e);
+        l1 = ld16_even(blk + 64 * n + 32 + e);
+        hi = ld16_even(blk + 128 + 32 * n + e);
+        sc = *reinterpret_cast<const Even8 *>(blk + 192 + 8 * n);
+        d = *reinterpret_cast<const uint16_t *>(blk + 208);
+    }
+};
+template <>
+struct WideRaw<kWQ8> {
+    Even8 q[8];       // codes 8 kg .. +7 of 32-element block j
+    uint32_t d;       // fp16 d of blocks 2 kg and 2 kg + 1
+    __device__ __forceinline__ void load(const uint8_t *blk, int kg) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) q[j] = *reinterpret_cast<const Even8 *>(blk + kQ8Bytes * j + 2 + 8 * kg);
+        d = (uint32_t) * reinterpret_cast<const uint16_t *>(blk + 2 * kQ8Bytes * kg) |
+            (uint32_t) * reinterpret_cast<const uint16_t *>(blk + 2 * kQ8Bytes * kg + kQ8Bytes) << 16;
+    }
+};
+
+// The operands made from them: digit planes of four 64-element fragments, and
+// the scales of the lane's four output rows 4 kg + i.
+template <int WK>
+struct WideOps;
+template <>
+struct WideOps<kWQ4> {
+    i32x4_t a[2][4];   // digit (8s, 1s), fragment 2 t + nibble
+    h4_t mins;
+    float dw[4], dmw[4];
+    // fragment f = (t, nibble) covers bytes 128 t + 64 (kg >> 1) + 32 nibble +
+    // 16 (kg & 1) .. +15 of the image block
+    static __device__ __forceinline__ int xoff(int f, int kg) {
+        return 128 * (f >> 1) + 64 * (kg >> 1) + 32 * (f & 1) + 16 * (kg & 1);
+    }
+    __device__ __forceinline__ void make(const WideRaw<kWQ4> &r, uint32_t *hdr, int kg, int rr) {
+        if (kg == 0) hdr[rr] = r.h.x;
+        const uint32_t u0 = r.h.y, u1 = r.h.z, u2 = r.h.w;
+        const uint32_t sc[2] = {u0 & 0x3f3f3f3fu, (u2 & 0x0f0f0f0fu) | ((u0 >> 2) & 0x30303030u)};
+        const uint32_t mn = (kg & 1) ? ((u2 >> 4) & 0x0f0f0f0fu) | ((u1 >> 2) & 0x30303030u)
+                                     : u1 & 0x3f3f3f3fu;
+        const float mw = kg < 2 ? 64.0f : 1.0f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mins[i] = (_Float16)((float)((mn >> (8 * i)) & 255u) * mw);
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {
+            const uint32_t s = (sc[f >> 1] >> (16 * (kg >> 1) + 8 * (f & 1))) & 255u;
+            const uint32_t sh = (s >> 3) * 0x10001u, sl = (s & 7u) * 0x10001u;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t w = r.q[f >> 1][k];
+                const uint32_t c = ((f & 1) ? w >> 4 : w) & 0x0f0f0f0fu;
+                a[0][f][k] = (int)pk_mul(c, sh);
+                a[1][f][k] = (int)pk_mul(c, sl);
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        const u32x4_t d = *reinterpret_cast<const u32x4_t *>(hdr + 4 * kg);
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            dw[i] = h2f(d[i] & 0xffffu);
+            dmw[i] = h2f(d[i] >> 16);
+        }
+    }
+    // one column tile: xc = the lane's column's codes in LDS, xa = its split
+    // 32-element sums (16 f16)
+    struct X {
+        i32x4_t b[4];
+        h4_t m;
+        float dx;
+    };
+    static __device__ __forceinline__ void load(X &x, const uint8_t *xc, const uint8_t *xa,
+                                                const float *xd, int kg) {
+#pragma unroll
+        for (int f = 0; f < 4; ++f) x.b[f] = *reinterpret_cast<const i32x4_t *>(xc + xoff(f, kg));
+        x.m = *reinterpret_cast<const h4_t *>(xa + 8 * kg);
+        x.dx = *xd;
+    }
+    __device__ __forceinline__ void add(const X &x, f4_t &acc) const {
+        i32x4_t h = {0, 0, 0, 0}, l = {0, 0, 0, 0};
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {
+            h = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0][f], x.b[f], h, 0, 0, 0);
+            l = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[1][f], x.b[f], l, 0, 0, 0);
+        }
+        const f4_t m = __builtin_amdgcn_mfma_f32_16x16x16f16(mins, x.m, f4_t{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            acc[i] = q4_block_term(dw[i], dmw[i], x.dx, (float)(h[i] * 8 + l[i]), m[i], acc[i]);
+    }
+};
+template <>
+struct WideOps<kWQ6> {
+    i32x4_t a[2][4];   // high and low byte of code x scale, fragment g
+    float dw[4];
+    static __device__ __forceinline__ int xoff(int g, int kg) {
+        return 128 * (kg >> 1) + 32 * g + 16 * (kg & 1);
+    }
+    __device__ __forceinline__ void make(const WideRaw<kWQ6> &r, uint32_t *hdr, int kg, int rr) {
+        if (kg == 0) hdr[rr] = r.d;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int s = (int)(int8_t)(r.sc.w[g >> 1] >> (16 * (g & 1) + 8 * (kg & 1)));
+            const uint32_t m = (uint32_t)(s & 0xffff) * 0x10001u;
+            const uint32_t c = (uint32_t)((128 - 32 * s) & 0xffff) * 0x10001u;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t l = (g & 1) ? r.l1[k] : r.l0[k], h = r.hi[k];
+                const uint32_t u = ((g < 2 ? l : l >> 4) & 0x0f0f0f0fu) |
+                                   ((g == 0 ? h << 4 : g == 1 ? h << 2 : g == 2 ? h : h >> 2) & 0x30303030u);
+                // 16 bits each: code x scale + 128 of the even and odd codes
+                const uint32_t pe = pk_mad(u & 0x00ff00ffu, m, c);
+                const uint32_t po = pk_mad((u >> 8) & 0x00ff00ffu, m, c);
+                a[0][g][k] = (int)__builtin_amdgcn_perm(po, pe, 0x07030501u);
+                a[1][g][k] = (int)(__builtin_amdgcn_perm(po, pe, 0x06020400u) ^ 0x80808080u);
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        const u32x4_t d = *reinterpret_cast<const u32x4_t *>(hdr + 4 * kg);
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dw[i] = h2f(d[i]);
+    }
+    struct X {
+        i32x4_t b[4];
+        float dx;
+    };
+    static __device__ __forceinline__ void load(X &x, const uint8_t *xc, const uint8_t *,
+                                                const float *xd, int kg) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) x.b[g] = *reinterpret_cast<const i32x4_t *>(xc + xoff(g, kg));
+        x.dx = *xd;
+    }
+    __device__ __forceinline__ void add(const X &x, f4_t &acc) const {
+        i32x4_t h = {0, 0, 0, 0}, l = {0, 0, 0, 0};
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            h = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[0][g], x.b[g], h, 0, 0, 0);
+            l = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[1][g], x.b[g], l, 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            acc[i] = q6_block_term(dw[i], x.dx, (float)(h[i] * 256 + l[i]), acc[i]);
+    }
+};
+template <>
+struct WideOps<kWQ8> {
+    uint64_t q[8];
+    u32x4_t dw[4];   // fp16 d of the rows' eight blocks
+    __device__ __forceinline__ void make(const WideRaw<kWQ8> &r, uint32_t *hdr, int kg, int rr) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) q[j] = ((uint64_t)r.q[j].w[1] << 32) | r.q[j].w[0];
+        hdr[4 * rr + kg] = r.d;
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dw[i] = *reinterpret_cast<const u32x4_t *>(hdr + 4 * (4 * kg + i));
+        __builtin_amdgcn_wave_barrier();
+    }
+    // xa: the column's 8 block scales (f32)
+    struct X {
+        uint64_t b[8];
+        f4_t d[2];
+    };
+    static __device__ __forceinline__ void load(X &x, const uint8_t *xc, const uint8_t *xa,
+                                                const float *, int kg) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x.b[j] = *reinterpret_cast<const uint64_t *>(xc + 32 * j + 8 * kg);
+        x.d[0] = reinterpret_cast<const f4_t *>(xa)[0];
+        x.d[1] = reinterpret_cast<const f4_t *>(xa)[1];
+    }
+    __device__ __forceinline__ void add(const X &x, f4_t &acc) const {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const i32x4_t c = mfma_i8(q[j], x.b[j], i32x4_t{0, 0, 0, 0});
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                acc[i] = fmaf((float)c[i], h2f((dw[i][j >> 1] >> (16 * (j & 1))) & 0xffffu) *
+                                               x.d[j >> 2][j & 3], acc[i]);
+        }
+    }
+};
+
+constexpr int kWideCol = 272;   // bytes per staged column: 256 codes, padded against bank conflicts
+
+// Two image blocks and the waves' block headers
+template <int CT, int NW>
+struct WideLds {
+    uint8_t codes[2][16 * CT * kWideCol];
+    uint8_t aux[2][16 * CT * 32];
+    float dx[2][16 * CT];
+    uint32_t hdr[NW][64];
+};
+
+template <int WK, int CT, int RT, bool SW>
+__device__ __forceinline__ void wide_body(const MmArgs &a, const MmOut &o0, const MmOut &o1,
+                                          WideLds<CT, (SW ? 2 : 1) * RT> &sm) {
+    constexpr int NT = 64 * RT * (SW ? 2 : 1);   // threads
+    constexpr int XI = 16 * CT * 16 / NT;        // 16-byte image pieces per thread
+    static_assert(NT * XI == 16 * CT * 16 && NT >= 16 * CT, "the work group stages whole blocks");
+    const int tid = threadIdx.x, lane = tid & 63, kg = lane >> 4, rr = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int K = a.n_in, nb = K >> 8, kw = a.kw;
+    constexpr int bbytes = WK == kWQ4 ? kQ4Bytes : WK == kWQ8 ? kQ8Per256 : kQ6Bytes;
+    // SwiGLU: the first RT waves take W1's rows, the others the same rows of W3
+    const int row0 = ((int)blockIdx.x - o0.tile0) * (16 * RT) + 16 * (wave % RT);
+    const int col0 = (int)blockIdx.y * 16 * CT;
+    const uint8_t *wp = (wave < RT ? o0.w : o1.w) + (int64_t)min(row0 + rr, o0.n_rows - 1) * nb * bbytes;
+
+    // the image block of the work group's columns: 16-byte pieces, piece
+    // (column, 4 q + g) holding codes 64 q + 8 g + e and 64 q + 32 + 8 g + e
+    // (k_q8k_rows' order); in LDS the codes are in their natural order
+    struct XPiece {
+        u32x4_t r[XI], s;
+        float d;
+    };
+    auto load_x = [&](XPiece &x, int b) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < XI; ++i) {
+            const int col = min(col0 + NT / 16 * i + (tid >> 4), a.n_cols - 1);
+            x.r[i] = *reinterpret_cast<const u32x4_t *>(a.xq + (int64_t)col * K + 256 * b + 16 * (tid & 15));
+        }
+        // (every thread loads: a load on one path only makes the wait counts
+        // assume it absent, and each wait then drains the others)
+        const int col = min(col0 + min(tid, 16 * CT - 1), a.n_cols - 1);
+        if (WK != kWQ6) x.s = *reinterpret_cast<const u32x4_t *>(a.xbs + (int64_t)col * (K / 32) + 8 * b);
+        if (WK != kWQ8) x.d = a.xd[(int64_t)col * nb + b];
+    };
+    auto store_x = [&](const XPiece &x, int buf) __attribute__((always_inline)) {
+        const int at = (tid >> 4) * kWideCol + 64 * ((tid >> 2) & 3) + 8 * (tid & 3);
+#pragma unroll
+        for (int i = 0; i < XI; ++i) {
+            uint8_t *p = &sm.codes[buf][NT / 16 * i * kWideCol + at];
+            *reinterpret_cast<u32x2_t *>(p) = u32x2_t{x.r[i].x, x.r[i].y};
+            *reinterpret_cast<u32x2_t *>(p + 32) = u32x2_t{x.r[i].z, x.r[i].w};
+        }
+        if (tid < 16 * CT) {
+            if (WK != kWQ8) sm.dx[buf][tid] = x.d;
+            if (WK == kWQ4) {
+                // s = 64 hi + lo, lo in 0 .. 63: both exact in f16
+                _Float16 *p = reinterpret_cast<_Float16 *>(&sm.aux[buf][32 * tid]);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const int w = (int)x.s[i >> 1];
+                    const int s = (i & 1) ? w >> 16 : (int)(int16_t)(w & 0xffff);
+                    p[i] = (_Float16)(float)(s >> 6);
+                    p[8 + i] = (_Float16)(float)(s & 63);
+                }
+            } else if (WK == kWQ8) {
+                float *p = reinterpret_cast<float *>(&sm.aux[buf][32 * tid]);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) p[i] = h2f((x.s[i >> 1] >> (16 * (i & 1))) & 0xffffu);
+            }
+        }
+    };
+
+    f4_t acc[CT], total[CT];
+#pragma unroll
+    for (int c = 0; c < CT; ++c) acc[c] = total[c] = f4_t{0, 0, 0, 0};
+    // blocks in k_gemm_kq's order: v, v + kw, .. of virtual wave v, then the
+    // next one's; past the last block, block 0 (requested, unused)
+    int ahead = 0, va = 0;
+    auto fetch = [&](WideRaw<WK> &r, XPiece &x) __attribute__((always_inline)) {
+        load_x(x, ahead);
+        r.load(wp + (int64_t)ahead * bbytes, kg);
+        ahead += kw;
+        if (ahead >= nb) ahead = ++va < nb ? va : 0;
+    };
+    // two blocks ahead in registers, two image blocks in LDS
+    WideRaw<WK> raw[2];
+    XPiece xp[2] = {};
+    fetch(raw[0], xp[0]);
+    fetch(raw[1], xp[1]);
+    store_x(xp[0], 0);
+    __syncthreads();
+    int b = 0, v = 0;   // the current block and its virtual wave
+    auto step = [&](WideRaw<WK> &rw, XPiece &xfree, const XPiece &xnext, int buf)
+                    __attribute__((always_inline)) {
+        using Ops = WideOps<WK>;
+        Ops op;
+        op.make(rw, sm.hdr[wave], kg, rr);
+        fetch(rw, xfree);
+        typename Ops::X x[2];
+        auto get = [&](typename Ops::X &d, int c) __attribute__((always_inline)) {
+            Ops::load(d, &sm.codes[buf][(16 * c + rr) * kWideCol], &sm.aux[buf][32 * (16 * c + rr)],
+                      &sm.dx[buf][16 * c + rr], kg);
+        };
+        get(x[0], 0);
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+            // the next column tile's operands are requested before this one's
+            // products: left to the compiler, each read was waited for alone
+            if (c + 1 < CT) get(x[(c + 1) & 1], c + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            op.add(x[c & 1], acc[c]);
+        }
+        b += kw;
+        if (b >= nb) {   // the virtual wave's last block
+            b = ++v;
+#pragma unroll
+            for (int c = 0; c < CT; ++c) {
+                total[c] += acc[c];
+                acc[c] = f4_t{0, 0, 0, 0};
+            }
+        }
+        store_x(xnext, buf ^ 1);
+        __syncthreads();
+    };
+    for (int it = 0; it + 1 < nb; it += 2) {
+        step(raw[0], xp[0], xp[1], 0);
+        step(raw[1], xp[1], xp[0], 1);
+    }
+    if (nb & 1) step(raw[0], xp[0], xp[1], 0);
+
+    f4_t up[SW ? CT : 1];   // W3's sums
+    if constexpr (SW) {
+        static_assert(sizeof(sm.codes) >= RT * CT * 64 * sizeof(f4_t), "exchanged in the code buffers");
+        f4_t *ex = reinterpret_cast<f4_t *>(&sm.codes[0][0]) + (wave % RT) * CT * 64 + lane;
+        if (wave >= RT) {
+#pragma unroll
+            for (int c = 0; c < CT; ++c) ex[64 * c] = total[c];
+        }
+        __syncthreads();
+        if (wave >= RT) return;
+#pragma unroll
+        for (int c = 0; c < CT; ++c) up[c] = ex[64 * c];
+    }
+
+    // outputs: lane (kg, n) holds rows row0 + 4 kg + i of input row n of each
+    // column tile; the same epilogue as k_gemm_kq
+    const int r0 = row0 + 4 * kg;
+    const bool v4 = (o0.n_rows & 3) == 0 && (reinterpret_cast<uintptr_t>(o0.y) & 15u) == 0;
+    float b0[4], b1[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int r = min(r0 + i, o0.n_rows - 1);
+        b0[i] = o0.bias ? o0.bias[r] : 0.0f;
+        b1[i] = SW && o1.bias ? o1.bias[r] : 0.0f;
+    }
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+        const int col = col0 + 16 * c + rr;
+        if (col >= a.n_cols || r0 >= o0.n_rows) continue;
+        const int64_t at = (int64_t)(a.y_ring > 0 ? (a.y_row0 + col) % a.y_ring : col) * o0.n_rows + r0;
+        float y[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) y[i] = o0.bias ? total[c][i] + b0[i] : total[c][i];
+        if constexpr (SW) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                y[i] = silu(y[i]) * (o1.bias ? up[c][i] + b1[i] : up[c][i]);
+        } else if (a.gelu) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) y[i] = gelu_erf(y[i]);
+        } else if (o0.rope) {
+#pragma unroll
+            for (int i = 0; i < 4; i += 2)
+                rope_pair(y[i], y[i + 1], ((r0 + i) % a.rope_hd) >> 1, (float)(a.rope_pos0 + col), a.rope_ts);
+        } else if (o0.add) {
+            if (v4 && (reinterpret_cast<uintptr_t>(o0.add) & 15u) == 0) {
+                const float4 r4 = *reinterpret_cast<const float4 *>(o0.add + at);
+                y[0] = r4.x + y[0];
+                y[1] = r4.y + y[1];
+                y[2] = r4.z + y[2];
+                y[3] = r4.w + y[3];
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (r0 + i < o0.n_rows) y[i] = o0.add[at + i] + y[i];
+            }
+        }
+        if (v4) {
+            *reinterpret_cast<float4 *>(o0.y + at) = make_float4(y[0], y[1], y[2], y[3]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (r0 + i < o0.n_rows) o0.y[at + i] = y[i];
+        }
+    }
+}
+
+template <int CT, int RT, bool SW, bool Q80>
+__global__ void __launch_bounds__(64 * RT * (SW ? 2 : 1), 2) k_gemm_wide(MmArgs a) {
+    __shared__ __align__(16) WideLds<CT, (SW ? 2 : 1) * RT> sm;
+    int seg = 0;
+    if constexpr (!SW) {
+#pragma unroll
+        for (int k = 1; k < kMvMaxOuts; ++k)
+            if (k < a.n_outs && (int)blockIdx.x >= a.out[k].tile0) seg = k;
+    }
+    const MmOut o0 = mm_out_at(a, seg);
+    const MmOut o1 = SW ? a.out[1] : o0;
+    if constexpr (Q80) wide_body<kWQ8, CT, RT, SW>(a, o0, o1, sm);
+    else if (o0.dtype == VKV_DTYPE_Q4_K) wide_body<kWQ4, CT, RT, SW>(a, o0, o1, sm);
+    else wide_body<kWQ6, CT, RT, SW>(a, o0, o1, sm);
+}
+
 }  // namespace
 
 hipError_t launch_matvec(const MvArgs &a, int n_wg, hipStream_t st) {
@@ -1812,7 +2307,66 @@ hipError_t launch_q8k_rows(const float *x, int64_t x_stride, int x_ring, int x_r
     return hipGetLastError();
 }
 
+namespace {
+// 64-row tiles x input columns (k_gemm_wide)
+template <int CT, int RT, bool SW>
+hipError_t launch_gemm_wide(MmArgs a, hipStream_t st) {
+    int tiles = 0, tiles16 = 0;
+    for (int k = 0; k < a.n_outs; ++k) {
+        if (a.swiglu && k == 1) {
+            a.out[1].tile0 = 0x7fffffff;   // W3 rides with W1's tiles
+            continue;
+        }
+        a.out[k].tile0 = tiles;
+        tiles += (a.out[k].n_rows + 16 * RT - 1) / (16 * RT);
+        tiles16 += (a.out[k].n_rows + 15) / 16;
+    }
+    for (int k = a.n_outs; k < kMvMaxOuts; ++k) a.out[k].tile0 = 0x7fffffff;
+    // k_gemm_kq's K split for these matrices
+    a.kw = (tiles16 < 128 ? 16 : 8) / (a.swiglu ? 2 : 1);
+    const dim3 g((unsigned)tiles, (unsigned)((a.n_cols + 16 * CT - 1) / (16 * CT)));
+    const bool q80 = a.out[0].dtype == VKV_DTYPE_Q8_0;
+    constexpr int NT = 64 * RT * (SW ? 2 : 1);
+    if (q80) k_gemm_wide<CT, RT, SW, true><<<g, NT, 0, st>>>(a);
+    else k_gemm_wide<CT, RT, SW, false><<<g, NT, 0, st>>>(a);
+    return hipGetLastError();
+}
+}  // namespace
+
 hipError_t launch_gemm_kq(MmArgs a, int n_col_tiles, hipStream_t st) {
+    // Many input rows: k_gemm_wide, the image read once per 64 (or 32) rows
+    // instead of once per 16.  It needs enough tiles: k_gemm_kq's waves split
+    // K, so it fills the chip with few.  Measured on MI355X (us, k_gemm_kq
+    // against k_gemm_wide) with T 16-row tiles and P input rows: T = 384,
+    // K = 3072 (Q/K/V): P = 38 19.7 / 21.5, 64 22.6 / 22.2, 128 35.7 / 25.1,
+    // 503 114 / 57; T = 192, K = 4096: 64 22.1 / 20.5, 96 29.6 / 21.2, 503
+    // 97 / 40; T = 192, K = 9216 (Q6_K): 64 38.6 / 40.9, 128 54.1 / 50.7, 503
+    // 180 / 95; T = 80, K = 2048: 64 12.5 / 13.9, 128 16.7 / 14.3; SwiGLU
+    // with T = 576: 20 30.3 / 22-23, 38 37.7 / 30, 503 299 / 119, T = 320:
+    // 20 13.7 / 12, 128 28.3 / 18.7.
+    if (!a.x && n_col_tiles > 1) {
+        int t16 = 0;
+        for (int k = 0; k < a.n_outs; ++k)
+            if (!(a.swiglu && k == 1)) t16 += (a.out[k].n_rows + 15) / 16;
+        const int64_t work = (int64_t)t16 * a.n_cols;
+        // (Q8_0, a float scale per 32 elements in both: from more tiles on;
+        // T = 576, SwiGLU: 38 51.6 / 62.6, 61 61.0 / 58.0, 503 368 / 206;
+        // T = 192: 128 33.4 / 38.5, 251 59.9 / 54.8)
+        const bool q80 = a.out[0].dtype == VKV_DTYPE_Q8_0;
+        if (a.swiglu) {
+            // two waves' rows x 64 inputs from 512 tiles of 16 x 64, else x 32
+            if (work >= 32768) return launch_gemm_wide<4, 2, true>(a, st);
+            if (work >= (q80 ? 24576 : 6144)) return launch_gemm_wide<2, 2, true>(a, st);
+        } else if (work >= (q80 ? 32768 : a.n_cols >= 96 ? 10240 : 16384)) {
+            // 64 inputs per work group while that leaves every SIMD a wave,
+            // else 32; then work groups of 4 waves where they are no more
+            // than the CUs, of 2 where those would leave CUs idle or double up
+            const int64_t w32 = (int64_t)t16 * ((a.n_cols + 31) / 32);
+            if ((int64_t)t16 * ((a.n_cols + 63) / 64) >= 1024) return launch_gemm_wide<4, 4, false>(a, st);
+            if (w32 > 512 && w32 <= 1024) return launch_gemm_wide<2, 4, false>(a, st);
+            return launch_gemm_wide<2, 2, false>(a, st);
+        }
+    }
     // the 16-row tiles of each matrix are consecutive work groups
     int tiles = 0;
     for (int k = 0; k < a.n_outs; ++k) {
@@ -1835,48 +2389,39 @@ hipError_t launch_gemm_kq(MmArgs a, int n_col_tiles, hipStream_t st) {
     // accumulators spills at four waves per SIMD, and measured slower.
     // A fused-input call (a.x) quantizes each work group's input rows into
     // dynamic LDS (the caller checked gemm_fused_lds).
-    const bool fq = a.x != nullptr;
-    const int cols = gemm_cols_per_wg(a, n_col_tiles);
-    const size_t lds = fq ? fused_lds_bytes(cols, a.n_in, a.norm_w != nullptr) : 0;
+    const bool fq = a.x != nullptr;   // (one column tile)
+    const size_t lds = fq ? fused_lds_bytes(16, a.n_in, a.norm_w != nullptr) : 0;
+    const dim3 g((unsigned)tiles, (unsigned)n_col_tiles);
     if (tiles < 128) {
-        const dim3 g((unsigned)tiles, (unsigned)n_col_tiles);
         if (fq) k_gemm_kq<16, 1, true><<<g, 1024, lds, st>>>(a);
         else k_gemm_kq<16, 1, false><<<g, 1024, 0, st>>>(a);
     } else if (n_col_tiles == 1) {
-        const dim3 g((unsigned)tiles, 1u);
         if (fq) k_gemm_kq<8, 1, true><<<g, 512, lds, st>>>(a);
         else k_gemm_kq<8, 1, false><<<g, 512, 0, st>>>(a);
     } else {
-        const dim3 g((unsigned)tiles, (unsigned)((n_col_tiles + 1) / 2));
-        if (fq) k_gemm_kq<8, 2, true><<<g, 512, lds, st>>>(a);
-        else k_gemm_kq<8, 2, false><<<g, 512, 0, st>>>(a);
+        k_gemm_kq<8, 2, false><<<dim3((unsigned)tiles, (unsigned)((n_col_tiles + 1) / 2)), 512, 0, st>>>(a);
     }
     return hipGetLastError();
 }
 
-int gemm_cols_per_wg(const MmArgs &a, int n_col_tiles) {
-    int tiles = 0;
-    for (int k = 0; k < a.n_outs; ++k)
-        if (!(a.swiglu && k == 1)) tiles += (a.out[k].n_rows + 15) / 16;
-    return (tiles < 128 || n_col_tiles == 1) ? 16 : 32;
-}
-
-// Whether the call's input image is quantized inside its work groups: every
-// 16-lane group then has at most kFqRounds (row, block) tasks (the realtime
-// encoder's 4-frame chunks, single adapter groups), and the image fits in LDS
-// beside the product's own.  Measured on MI355X: 16-frame encoder chunks
-// and 38-row prompts, with 3 to 12 tasks per group, run slower fused than
-// with the separate k_q8k_rows launch (2.68 vs 2.23 ms, 6.65 vs 3.40 ms).
-bool gemm_fused_ok(const MmArgs &a, int n_col_tiles) {
+// Whether the call's input image is quantized inside its work groups: at most
+// kFqRows input rows (the realtime encoder's 4-frame chunks, single adapter
+// groups), every 16-lane group with at most kFqRounds (row, block) tasks, and
+// the image in LDS beside the product's own.  Measured on MI355X against the
+// separate k_q8k_rows launch, with 16-row tiles T of K inputs: 4 rows T = 80,
+// K = 5120 10.4 against 11.7 us, T = 192, K = 4096 8.6 against 9.8, T = 384,
+// K = 1280 9.4 against 9.0; 8 rows 9.1 against 8.3 (T = 80, K = 2048) and
+// 11.2 against 9.1 (T = 384, K = 1280); 16 rows 12.4 against 8.9 (T = 80, K =
+// 2048), and with several column tiles every one of them quantized again.
+constexpr int kFqRows = 4;
+bool gemm_fused_ok(const MmArgs &a) {
     int tiles = 0;
     for (int k = 0; k < a.n_outs; ++k)
         if (!(a.swiglu && k == 1)) tiles += (a.out[k].n_rows + 15) / 16;
     const int waves = tiles < 128 ? 16 : 8;
-    const int cols = gemm_cols_per_wg(a, n_col_tiles);
-    const int rows = std::min(cols, a.n_cols);
-    return rows * (a.n_in / 256) <= kFqRounds * 4 * waves &&
+    return a.n_cols <= kFqRows && a.n_cols * (a.n_in / 256) <= kFqRounds * 4 * waves &&
            (!a.norm_w || a.n_in <= kFqNormPer * 64 * waves) &&
-           fused_lds_bytes(cols, a.n_in, a.norm_w != nullptr) <= 128 * 1024;
+           fused_lds_bytes(16, a.n_in, a.norm_w != nullptr) <= 128 * 1024;
 }
 
 hipError_t launch_rms_norm_rows(const float *x, int n_rows, int n, const float *w, const float *b,
