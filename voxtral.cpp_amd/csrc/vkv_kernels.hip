@@ -2180,7 +2180,51 @@ __global__ void __launch_bounds__(256) k_window_merge(const float *part_o, const
 // ---------------------------------------------------------------------------
 // SPL > 1: keys split over SPL work groups per (head, tile), as in
 // k_window_mfma (partials merged by k_window_merge; GQA 1 only).
-template <int D, int W, int SPL = 1>
+//
+// Q8: the same over a q8_0 cache, each value dequantised to f32 exactly
+// (code x fp16 d) on its way into the operand, so every product and sum stays
+// in f32 as on the scalar ALU (k_window, two passes over the keys with a
+// lane per key: a 199-token prefill over 237 keys took 213 us with its append,
+// this 21).  A
+// lane's run of dims is a block (D = 128) or half of one (D = 64).
+
+// A lane's run of DL dims of one K or V row, four at a time as f32.
+template <int DL, bool Q8>
+struct WinRow;
+template <int DL>
+struct WinRow<DL, false> {
+    float4 r[DL / 4];
+    __device__ __forceinline__ void load(const uint8_t *p, int t) {
+        r[t] = reinterpret_cast<const float4 *>(p)[t];
+    }
+    __device__ __forceinline__ float4 at(int t) const { return r[t]; }
+};
+template <int DL>
+struct WinRow<DL, true> {
+    struct __attribute__((packed, aligned(2))) Codes {   // blocks are 2-byte aligned
+        uint32_t w[4];
+    };
+    uint32_t c[DL / 4];
+    uint32_t d;
+    // codes at p; the block's fp16 d before its first code
+    __device__ __forceinline__ void load(const uint8_t *p, const uint8_t *pd) {
+#pragma unroll
+        for (int t = 0; t < DL / 16; ++t) {
+            const Codes v = *reinterpret_cast<const Codes *>(p + 16 * t);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) c[4 * t + i] = v.w[i];
+        }
+        d = *reinterpret_cast<const uint16_t *>(pd);
+    }
+    __device__ __forceinline__ float4 at(int t) const {
+        const float s = (float)__builtin_bit_cast(_Float16, (uint16_t)d);
+        const uint32_t w = c[t];
+        return make_float4((float)(int8_t)w * s, (float)(int8_t)(w >> 8) * s,
+                           (float)(int8_t)(w >> 16) * s, (float)(int8_t)(w >> 24) * s);
+    }
+};
+
+template <int D, int W, int SPL = 1, bool Q8 = false>
 __device__ __forceinline__ void window_mfma_f32(const WindowArgs &a) {
     constexpr int DL = D / 4;           // contiguous head dims per lane
     constexpr int NT = D / 16;          // 16-dim tiles of P.V
@@ -2240,25 +2284,34 @@ __device__ __forceinline__ void window_mfma_f32(const WindowArgs &a) {
 
     // K and V of key jb + lr, dims [DL lg, +DL): one contiguous run per lane;
     // indices clamp into [j_lo, j_hi) (keys outside it are masked)
-    auto load_kv = [&](int jb, float4 (&kr)[DL / 4], float4 (&vr)[DL / 4]) __attribute__((always_inline)) {
+    using Row = WinRow<DL, Q8>;
+    auto load_kv = [&](int jb, Row &kr, Row &vr) __attribute__((always_inline)) {
         const int jk = max(min(jb + lr, j_hi - 1), j_lo);
         // an empty key range reads slot 0 (unused)
-        const uint32_t off = (uint32_t)(j_lo < j_hi ? slot_of(a.seg, jk) : 0) * (uint32_t)a.row_bytes +
-                             (uint32_t)(g * D + DL * lg) * 4u;
+        const uint32_t row = (uint32_t)(j_lo < j_hi ? slot_of(a.seg, jk) : 0) * (uint32_t)a.row_bytes;
+        if constexpr (Q8) {
+            const uint32_t dim = (uint32_t)(g * D + DL * lg);
+            const uint32_t blk = row + (dim >> 5) * 34u, off = blk + 2u + (dim & 31u);
+            kr.load(kl + off, kl + blk);
+            vr.load(vl + off, vl + blk);
+        } else {
+            const uint32_t off = row + (uint32_t)(g * D + DL * lg) * 4u;
 #pragma unroll
-        for (int t = 0; t < DL / 4; ++t) {
-            kr[t] = reinterpret_cast<const float4 *>(kl + off)[t];
-            vr[t] = reinterpret_cast<const float4 *>(vl + off)[t];
+            for (int t = 0; t < DL / 4; ++t) {
+                kr.load(kl + off, t);
+                vr.load(vl + off, t);
+            }
         }
     };
-    auto process = [&](const float4 (&kr)[DL / 4], const float4 (&vr)[DL / 4], int jb) __attribute__((always_inline)) {
+    auto process = [&](const Row &kr, const Row &vr, int jb) __attribute__((always_inline)) {
         // V^T tile: this lane's key lr, dims DL lg + x
 #pragma unroll
         for (int t = 0; t < DL / 4; ++t) {
-            vt[(DL * lg + 4 * t + 0) * VS + lr] = vr[t].x;
-            vt[(DL * lg + 4 * t + 1) * VS + lr] = vr[t].y;
-            vt[(DL * lg + 4 * t + 2) * VS + lr] = vr[t].z;
-            vt[(DL * lg + 4 * t + 3) * VS + lr] = vr[t].w;
+            const float4 v4 = vr.at(t);
+            vt[(DL * lg + 4 * t + 0) * VS + lr] = v4.x;
+            vt[(DL * lg + 4 * t + 1) * VS + lr] = v4.y;
+            vt[(DL * lg + 4 * t + 2) * VS + lr] = v4.z;
+            vt[(DL * lg + 4 * t + 3) * VS + lr] = v4.w;
         }
         // S^T = K Q^T, one MFMA per dim step, into four independent
         // accumulators (dims = 0, 1, 2, 3 mod 4) summed at the end: one
@@ -2267,10 +2320,11 @@ __device__ __forceinline__ void window_mfma_f32(const WindowArgs &a) {
                           float4_t{0, 0, 0, 0}};
 #pragma unroll
         for (int t = 0; t < DL / 4; ++t) {
-            sa[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[t].x, qf[4 * t], sa[0], 0, 0, 0);
-            sa[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[t].y, qf[4 * t + 1], sa[1], 0, 0, 0);
-            sa[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[t].z, qf[4 * t + 2], sa[2], 0, 0, 0);
-            sa[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[t].w, qf[4 * t + 3], sa[3], 0, 0, 0);
+            const float4 k4 = kr.at(t);
+            sa[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.x, qf[4 * t], sa[0], 0, 0, 0);
+            sa[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.y, qf[4 * t + 1], sa[1], 0, 0, 0);
+            sa[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.z, qf[4 * t + 2], sa[2], 0, 0, 0);
+            sa[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.w, qf[4 * t + 3], sa[3], 0, 0, 0);
         }
         const float4_t st = (sa[0] + sa[1]) + (sa[2] + sa[3]);
         // lane holds keys jb + 4 lg + i (i = 0..3) for row lr
@@ -2303,6 +2357,26 @@ __device__ __forceinline__ void window_mfma_f32(const WindowArgs &a) {
             l += p[i];
         }
         __builtin_amdgcn_wave_barrier();
+        if constexpr (Q8) {
+            // A row stored from values beyond the format (infinite or NaN
+            // scale) must not reach the rows that mask it, whose zero weights
+            // the matrix core would still multiply by it: such a block is
+            // added on the vector ALU, each row its own keys.
+            if (__any((vr.d & 0x7c00u) == 0x7c00u)) {
+                for (int key = 0; key < 16; ++key) {
+                    const float sk = __shfl(sc[key & 3], 16 * (key >> 2) + lr);
+                    const float pk = __shfl(p[key & 3], 16 * (key >> 2) + lr);
+                    if (sk == -INFINITY) continue;
+#pragma unroll
+                    for (int T = 0; T < NT; ++T)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            o[T][e] = fmaf(pk, vt[(16 * T + 4 * lg + e) * VS + key], o[T][e]);
+                }
+                __builtin_amdgcn_wave_barrier();
+                return;
+            }
+        }
         // O^T tile T += V^T[16 T + lr][key 4 lg + s] p_s
 #pragma unroll
         for (int T = 0; T < NT; ++T)
@@ -2312,7 +2386,7 @@ __device__ __forceinline__ void window_mfma_f32(const WindowArgs &a) {
                                                              o[T], 0, 0, 0);
         __builtin_amdgcn_wave_barrier();
     };
-    float4 ka_[DL / 4], va_[DL / 4], kb_[DL / 4], vb_[DL / 4];
+    Row ka_, va_, kb_, vb_;
     // The block grid is absolute: wave w takes the 16-key blocks starting at
     // key positions = 16 w (mod 16 W), whatever the run's first query, so a
     // row meets its keys in the same blocks, waves and order under every
@@ -2327,18 +2401,34 @@ __device__ __forceinline__ void window_mfma_f32(const WindowArgs &a) {
         const int64_t src0 = (int64_t)layer * a.n_new * kv_dim;
         uint8_t *kw = a.k_w + (int64_t)layer * a.layer_bytes;
         uint8_t *vw = a.v_w + (int64_t)layer * a.layer_bytes;
-        for (int t = threadIdx.x; t < a.n_new * (D / 4); t += 64 * W) {
-            const int row = t / (D / 4);
+        // F32: 4 dims per thread; q8_0: 8, a quad per block (whole blocks per
+        // row, so a quad's threads leave the loop together)
+        constexpr int TD = Q8 ? 8 : 4;
+        for (int t = threadIdx.x; t < a.n_new * (D / TD); t += 64 * W) {
+            const int row = t / (D / TD);
             // split tiles: each new row is written by the work group whose
             // key blocks hold it, the only one that reads it
             if (SPL > 1 &&
                 (int)(((a.key_pos0 + n_keys - a.n_new + row) >> 4) % VW) / W != split)
                 continue;
-            const int col = g * D + (t % (D / 4)) * 4;
+            const int col = g * D + (t % (D / TD)) * TD;
             const int64_t so = src0 + (int64_t)row * kv_dim + col;
-            const int64_t dst = (int64_t)slot_of(a.wseg, row) * a.row_bytes + (int64_t)col * 4;
-            *reinterpret_cast<float4 *>(kw + dst) = *reinterpret_cast<const float4 *>(a.k_new + so);
-            *reinterpret_cast<float4 *>(vw + dst) = *reinterpret_cast<const float4 *>(a.v_new + so);
+            const int64_t dst = (int64_t)slot_of(a.wseg, row) * a.row_bytes;
+            if constexpr (Q8) {
+                float xk[8], xv[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    xk[e] = a.k_new[so + e];
+                    xv[e] = a.v_new[so + e];
+                }
+                store_new<FmtQ8>(kw + dst, col, xk, true);
+                store_new<FmtQ8>(vw + dst, col, xv, true);
+            } else {
+                *reinterpret_cast<float4 *>(kw + dst + (int64_t)col * 4) =
+                    *reinterpret_cast<const float4 *>(a.k_new + so);
+                *reinterpret_cast<float4 *>(vw + dst + (int64_t)col * 4) =
+                    *reinterpret_cast<const float4 *>(a.v_new + so);
+            }
         }
         __syncthreads();
     }
@@ -2419,6 +2509,18 @@ __global__ void __launch_bounds__(256) k_window_mfma_f32_128(WindowArgs a) {
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4)))
 k_window_mfma_f32_64_split(WindowArgs a) {
     window_mfma_f32<64, 4, kWinSplit>(a);
+}
+// the same over a q8_0 cache
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4)))
+k_window_mfma_q8_64(WindowArgs a) {
+    window_mfma_f32<64, 4, 1, true>(a);
+}
+__global__ void __launch_bounds__(256) k_window_mfma_q8_128(WindowArgs a) {
+    window_mfma_f32<128, 4, 1, true>(a);
+}
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4)))
+k_window_mfma_q8_64_split(WindowArgs a) {
+    window_mfma_f32<64, 4, kWinSplit, true>(a);
 }
 
 // ---------------------------------------------------------------------------
@@ -2615,8 +2717,7 @@ hipError_t launch_combine(const CombineArgs &a, int n_streams, hipStream_t st) {
 // valu: the scalar-ALU kernel instead of the matrix-core tile (cross-check and
 // A/B measurement)
 hipError_t launch_window(int dtype, bool valu, const WindowArgs &a_in, hipStream_t st) {
-    const bool mfma = (dtype == VKV_DTYPE_F16 || dtype == VKV_DTYPE_F32) && !valu &&
-                      (a_in.head_dim == 64 || a_in.head_dim == 128);
+    const bool mfma = !valu && (a_in.head_dim == 64 || a_in.head_dim == 128);
     WindowArgs a = a_in;
     // Every query tile of a kv head stores that head's new rows in the fused
     // write, so its bytes grow with tiles x rows: keep it for calls with few
@@ -2674,6 +2775,8 @@ hipError_t launch_window(int dtype, bool valu, const WindowArgs &a_in, hipStream
                 const dim3 gs((unsigned)(nt * a.n_kv_heads), 1u, (unsigned)kWinSplit);
                 if (dtype == VKV_DTYPE_F32)
                     hipLaunchKernelGGL(k_window_mfma_f32_64_split, gs, dim3(256), 0, st, b);
+                else if (dtype == VKV_DTYPE_Q8_0)
+                    hipLaunchKernelGGL(k_window_mfma_q8_64_split, gs, dim3(256), 0, st, b);
                 else
                     hipLaunchKernelGGL((k_window_mfma<64, 4, 1, kWinSplit>), gs, dim3(256), 0, st, b);
                 const int64_t n_vec = (int64_t)std::min(16 * nt, n_rows - 16 * t0) * a.n_q_heads;
@@ -2687,6 +2790,9 @@ hipError_t launch_window(int dtype, bool valu, const WindowArgs &a_in, hipStream
             // slower here: 18.3 against 17.6 us per 4-frame call)
             if (a.head_dim == 64) hipLaunchKernelGGL(k_window_mfma_f32_64, g2, dim3(256), 0, st, a);
             else hipLaunchKernelGGL(k_window_mfma_f32_128, g2, dim3(256), 0, st, a);
+        } else if (dtype == VKV_DTYPE_Q8_0) {
+            if (a.head_dim == 64) hipLaunchKernelGGL(k_window_mfma_q8_64, g2, dim3(256), 0, st, a);
+            else hipLaunchKernelGGL(k_window_mfma_q8_128, g2, dim3(256), 0, st, a);
         } else if (a.n_layers == 1 && a.head_dim == 64) {
             // a per-layer call without room for the split partials: 32 work
             // groups of 8 waves
