@@ -1765,27 +1765,29 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))
 
 // ---------------------------------------------------------------------------
 // The same products for many input rows.  k_gemm_kq gives each 16-row tile its
-// own work group, which reads the whole input image again; from about
-// kWideCols input rows that re-reading from L2 is what it spends its time on.
-// Here a work group owns 64 weight rows x 16 CT input rows: wave w rows
-// [16 w, 16 w + 16), every wave the same input columns, whose image block is
-// staged in LDS once per K block (double-buffered, one barrier per block; the
-// next block's weights and image are requested before the current one's
-// products).
+// own work group, which reads the whole input image again: at 503 input rows
+// Q/K/V (6144 x 3072) took 114 us, W1/W3 298 us, an eighth of the int8 rate's
+// share.  Here a work group owns 16 RT weight rows x 16 CT input rows: wave w
+// rows [16 w, 16 w + 16), every wave the same input columns, whose image block
+// is staged in LDS once per K block (double-buffered, one barrier per block).
+// The same calls take 47 and 107 us; bound by the ~5 VALU operations that an
+// output takes per block and those that make the operands (VALU ~5 clocks an
+// operation beside 16 for a product, measured), then by the few waves that
+// 3072-row matrices leave (one or two per SIMD).
 //
 // Products per 256-block.  The 6-bit scales are folded into the int8 operand
 // instead of multiplying each 32-element sum on the VALU, which took ~70 of
 // the ~90 VALU operations per tile and block: a Q4_K code times 3 bits of its
 // scale fits int8 (15 x 7), so with sc = 8 h + l the block's sum is
 // 8 sum (q h) x + sum (q l) x, two chains of four v_mfma_i32_16x16x64_i8; a
-// Q6_K code (-32 .. 31) times a digit of -3 .. 3 does too, and an int8 scale
-// is 49 a + 7 b + c with such digits: three chains.  The mins' sum is one
-// v_mfma_f32_16x16x16_f16: mins (and 64 mins) against the 32-element sums
-// split into 6 low bits and the rest, all integers that f16 holds, summed
-// below 2^24.  Every sum is the exact integer, and the blocks are added in
-// k_gemm_kq's order (virtual wave v of a.kw: blocks v, v + kw, ..; then the
-// waves in order), so both kernels give the same bits.  Q8_0 blocks have a
-// float scale per 32 elements: one v_mfma_i32_16x16x32_i8 each.
+// Q6_K code (-32 .. 31) times its int8 scale fits 16 bits, whose two bytes
+// are the chains' operands.  The mins' sum is one v_mfma_f32_16x16x16_f16:
+// mins (and 64 mins) against the 32-element sums split into 6 low bits and
+// the rest, all integers that f16 holds, summed below 2^24.  Every sum is the
+// exact integer, and the blocks are added in k_gemm_kq's order (virtual wave
+// v of a.kw: blocks v, v + kw, ..; then the waves in order), so both kernels
+// give the same bits.  Q8_0 blocks have a float scale per 32 elements: one
+// v_mfma_i32_16x16x32_i8 each.
 // ---------------------------------------------------------------------------
 typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 h4_t __attribute__((ext_vector_type(4)));
@@ -2022,6 +2024,12 @@ struct WideOps<kWQ8> {
 
 constexpr int kWideCol = 272;   // bytes per staged column: 256 codes, padded against bank conflicts
 
+// Blocks requested ahead: two where the launch rule leaves a SIMD one wave
+// (4 waves x 32 inputs; K = 9216, 128 inputs: 49.8 us against 55.3), else one,
+// whose registers leave room for a third wave per SIMD (503 inputs, K = 3072:
+// 47.9 us against 57.4 for Q/K/V, 111 against 121 for W1/W3).
+__host__ __device__ constexpr int wide_pre(int ct, int rt) { return ct == 2 && rt == 4 ? 2 : 1; }
+
 // Two image blocks and the waves' block headers
 template <int CT, int NW>
 struct WideLds {
@@ -2105,11 +2113,12 @@ __device__ __forceinline__ void wide_body(const MmArgs &a, const MmOut &o0, cons
         ahead += kw;
         if (ahead >= nb) ahead = ++va < nb ? va : 0;
     };
-    // two blocks ahead in registers, two image blocks in LDS
-    WideRaw<WK> raw[2];
-    XPiece xp[2] = {};
-    fetch(raw[0], xp[0]);
-    fetch(raw[1], xp[1]);
+    // PRE blocks ahead in registers, two image blocks in LDS
+    constexpr int PRE = wide_pre(CT, RT);
+    WideRaw<WK> raw[PRE];
+    XPiece xp[PRE] = {};
+#pragma unroll
+    for (int i = 0; i < PRE; ++i) fetch(raw[i], xp[i]);
     store_x(xp[0], 0);
     __syncthreads();
     int b = 0, v = 0;   // the current block and its virtual wave
@@ -2119,19 +2128,20 @@ __device__ __forceinline__ void wide_body(const MmArgs &a, const MmOut &o0, cons
         Ops op;
         op.make(rw, sm.hdr[wave], kg, rr);
         fetch(rw, xfree);
-        typename Ops::X x[2];
         auto get = [&](typename Ops::X &d, int c) __attribute__((always_inline)) {
             Ops::load(d, &sm.codes[buf][(16 * c + rr) * kWideCol], &sm.aux[buf][32 * (16 * c + rr)],
                       &sm.dx[buf][16 * c + rr], kg);
         };
-        get(x[0], 0);
+        typename Ops::X x[PRE];
+        if (PRE == 2) get(x[0], 0);
 #pragma unroll
         for (int c = 0; c < CT; ++c) {
-            // the next column tile's operands are requested before this one's
-            // products: left to the compiler, each read was waited for alone
-            if (c + 1 < CT) get(x[(c + 1) & 1], c + 1);
+            // one block ahead: a column tile's operands at a time (registers);
+            // two: the next tile's requested before this one's products
+            if (PRE == 1) get(x[0], c);
+            else if (c + 1 < CT) get(x[(c + 1) & 1], c + 1);
             __builtin_amdgcn_sched_barrier(0);
-            op.add(x[c & 1], acc[c]);
+            op.add(x[PRE == 1 ? 0 : c & 1], acc[c]);
         }
         b += kw;
         if (b >= nb) {   // the virtual wave's last block
@@ -2145,11 +2155,15 @@ __device__ __forceinline__ void wide_body(const MmArgs &a, const MmOut &o0, cons
         store_x(xnext, buf ^ 1);
         __syncthreads();
     };
-    for (int it = 0; it + 1 < nb; it += 2) {
-        step(raw[0], xp[0], xp[1], 0);
-        step(raw[1], xp[1], xp[0], 1);
+    if constexpr (PRE == 1) {
+        for (int it = 0; it < nb; ++it) step(raw[0], xp[0], xp[0], it & 1);
+    } else {
+        for (int it = 0; it + 1 < nb; it += 2) {
+            step(raw[0], xp[0], xp[1], 0);
+            step(raw[1], xp[1], xp[0], 1);
+        }
+        if (nb & 1) step(raw[0], xp[0], xp[1], 0);
     }
-    if (nb & 1) step(raw[0], xp[0], xp[1], 0);
 
     f4_t up[SW ? CT : 1];   // W3's sums
     if constexpr (SW) {
@@ -2219,7 +2233,7 @@ __device__ __forceinline__ void wide_body(const MmArgs &a, const MmOut &o0, cons
 }
 
 template <int CT, int RT, bool SW, bool Q80>
-__global__ void __launch_bounds__(64 * RT * (SW ? 2 : 1), 2) k_gemm_wide(MmArgs a) {
+__global__ void __launch_bounds__(64 * RT * (SW ? 2 : 1), wide_pre(CT, RT) == 1 ? 3 : 2) k_gemm_wide(MmArgs a) {
     __shared__ __align__(16) WideLds<CT, (SW ? 2 : 1) * RT> sm;
     int seg = 0;
     if constexpr (!SW) {
