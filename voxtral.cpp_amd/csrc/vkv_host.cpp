@@ -1250,12 +1250,12 @@ struct RowMap {
 };
 
 // RoPE of the outputs whose bit is set in mask (ggml mode 0, head_dim-wide
-// heads, position pos0 + input row), fused into the products' epilogue
+// heads, tab: the input rows' (cos, sin) pairs), fused into the products'
+// epilogue
 struct MmRope {
     uint32_t mask = 0;
     int32_t head_dim = 0;
-    int64_t pos0 = 0;
-    float theta = 0.0f;
+    const float2 *tab = nullptr;
 };
 
 vkv_status matmul_impl(const float *x, int32_t n_cols, int64_t n_in, const float *norm_w,
@@ -1383,9 +1383,8 @@ vkv_status matmul_impl(const float *x, int32_t n_cols, int64_t n_in, const float
                 return fail(VKV_STATUS_INVALID_ARGUMENT, "matmul: RoPE output %d shape", k);
             a.out[k].rope = 1;
         }
-        a.rope_ts = rope_theta_scale(rope.theta, rope.head_dim);
+        a.rope_tab = rope.tab;
         a.rope_hd = rope.head_dim;
-        a.rope_pos0 = rope.pos0;
     }
     e = launch_gemm_kq(a, n_col_tiles, as_stream(hip_stream));
     if (e != hipSuccess) return hip_fail(e, "matmul launch");
@@ -1637,6 +1636,7 @@ namespace {
 struct PromptBuffers {
     float *x, *q, *k, *v, *attn, *ffn;
     unsigned long long *amax;
+    float2 *rope;   // the rows' (cos, sin) pairs
     void *image;
     size_t image_bytes, bytes;
 };
@@ -1657,6 +1657,7 @@ PromptBuffers prompt_buffers(const vkv_dec_model &m, int32_t n, uint8_t *base) {
     t.attn = (float *)take((size_t)n * qd * 4);
     t.ffn = (float *)take((size_t)n * m.hidden * 4);
     t.amax = (unsigned long long *)take(16);
+    t.rope = (float2 *)take((size_t)n * (m.head_dim / 2) * sizeof(float2));
     // the products' Q8_K input image, sized for the widest input
     t.image_bytes = vkv_matmul_workspace(n, std::max<int64_t>(std::max<int64_t>(m.dim, m.hidden), qd));
     t.image = take(t.image_bytes);
@@ -1736,16 +1737,20 @@ vkv_status vkv_decoder_prompt(vkv_cache *cache, int32_t stream, vkv_ring *ring,
                                          t.x + (size_t)c0 * m.dim, st, c0 == 0 ? t.amax : nullptr);
         if (e != hipSuccess) return hip_fail(e, "decoder prompt: embedding launch");
     }
+    MmRope rope;
+    rope.mask = 3u;
+    rope.head_dim = m.head_dim;
+    rope.tab = t.rope;
+    {
+        hipError_t e = launch_rope_pairs(t.rope, n_tokens, m.head_dim / 2, pos0,
+                                         rope_theta_scale(m.rope_theta, m.head_dim), st);
+        if (e != hipSuccess) return hip_fail(e, "decoder prompt: rope launch");
+    }
     for (int32_t l = 0; l < m.n_layers; ++l) {
         const vkv_dec_layer &L = m.layers[l];
         const vkv_mm_out qkv[3] = {{L.attn_q, L.attn_q_type, qd, t.q, nullptr, nullptr},
                                    {L.attn_k, L.attn_k_type, kd, t.k, nullptr, nullptr},
                                    {L.attn_v, L.attn_v_type, kd, t.v, nullptr, nullptr}};
-        MmRope rope;
-        rope.mask = 3u;
-        rope.head_dim = m.head_dim;
-        rope.pos0 = pos0;
-        rope.theta = m.rope_theta;
         if (vkv_status s = matmul_impl(t.x, n_tokens, m.dim, L.attn_norm, nullptr, nullptr,
                                        m.norm_eps, qkv, 3, VKV_MV_STORE, t.image, t.image_bytes, hs,
                                        RowMap{}, RowMap{}, rope))
@@ -1877,6 +1882,7 @@ namespace {
 
 struct EncBuffers {
     float *qk, *v, *attn, *ffn;   // qk: q rows [n_new][qd] then k rows [n_new][kvd]
+    float2 *rope;                 // the frames' (cos, sin) pairs
     uint8_t *image;               // vkv_matmul workspace
     size_t image_bytes, bytes;
 };
@@ -1894,6 +1900,7 @@ EncBuffers enc_buffers(const vkv_enc_model &m, int32_t kvd, int32_t n_new, uint8
     t.v = (float *)take(rows * (size_t)kvd * 4);
     t.attn = (float *)take(rows * qd * 4);
     t.ffn = (float *)take(rows * m.hidden * 4);
+    t.rope = (float2 *)take(rows * (m.head_dim / 2) * sizeof(float2));
     t.image_bytes = std::max({vkv_matmul_workspace(n_new, m.dim), vkv_matmul_workspace(n_new, (int64_t)qd),
                               vkv_matmul_workspace(n_new, m.hidden)});
     t.image = take(t.image_bytes);
@@ -1957,18 +1964,22 @@ vkv_status encoder_chunk_impl(vkv_cache *cache, int32_t stream, const vkv_enc_pl
                     workspace_bytes, t.bytes);
     const float scale = 1.0f / std::sqrt((float)m.head_dim);
     float *q = t.qk, *k = t.qk + (size_t)N * qd;
+    // RoPE of the q and k rows at positions q_start + r, in the products'
+    // epilogue (vkv_rope's arithmetic, so the same bits)
+    MmRope rope;
+    rope.mask = 3u;
+    rope.head_dim = m.head_dim;
+    rope.tab = t.rope;
+    {
+        hipError_t e = launch_rope_pairs(t.rope, N, m.head_dim / 2, plan->q_start,
+                                         rope_theta_scale(m.rope_theta, m.head_dim), as_stream(hip_stream));
+        if (e != hipSuccess) return hip_fail(e, "encoder chunk: rope launch");
+    }
     for (int32_t l = 0; l < m.n_layers; ++l) {
         const vkv_enc_layer &L = m.layers[l];
         const vkv_mm_out qkv[3] = {{L.attn_q, L.attn_q_type, qd, q, nullptr, L.attn_q_b},
                                    {L.attn_k, L.attn_k_type, kvd, k, nullptr, nullptr},
                                    {L.attn_v, L.attn_v_type, kvd, t.v, nullptr, L.attn_v_b}};
-        // RoPE of the q and k rows at positions q_start + r, in the
-        // products' epilogue (vkv_rope's arithmetic, so the same bits)
-        MmRope rope;
-        rope.mask = 3u;
-        rope.head_dim = m.head_dim;
-        rope.pos0 = plan->q_start;
-        rope.theta = m.rope_theta;
         if (vkv_status s = matmul_impl(x, N, m.dim, L.attn_norm, L.attn_norm_b, nullptr, m.norm_eps,
                                        qkv, 3, VKV_MV_STORE, t.image, t.image_bytes, hip_stream,
                                        RowMap{}, RowMap{}, rope))

@@ -190,11 +190,9 @@ struct MmArgs {
     // y_ring > 0 (rows of a ring buffer), else p.
     int32_t y_ring, y_row0;
     // RoPE of the outputs with MmOut::rope: pairs (2i, 2i+1) of each
-    // rope_hd-wide head at position rope_pos0 + input row, angle
-    // pos * rope_ts^i (vkv_rope's arithmetic)
-    float rope_ts;
+    // rope_hd-wide head by input row p's (cos, sin), rope_tab[p][rope_hd / 2]
+    const float2 *rope_tab;
     int32_t rope_hd;
-    int64_t rope_pos0;
     // k_gemm_wide: the waves that k_gemm_kq splits K over for these matrices
     // (set by launch_gemm_kq)
     int32_t kw;
@@ -226,6 +224,8 @@ hipError_t launch_embed_rows(int dtype, const uint8_t *table, int64_t row_bytes,
                              const EmbedTokens &tok, int n_rows, int64_t n, const float *add,
                              int add_ring, int add_row0, float *y, hipStream_t st,
                              unsigned long long *zero_words = nullptr);
+// the (cos, sin) pairs of positions pos0 .. pos0 + n - 1, [n][pairs]
+hipError_t launch_rope_pairs(float2 *tab, int n, int pairs, int64_t pos0, float theta_scale, hipStream_t st);
 hipError_t launch_argmax(const float *x, int n, int32_t *out, hipStream_t st);
 // w_type: VKV_DTYPE_F32, _F16 or _Q8_0 (n_in % 32 == 0)
 hipError_t launch_rows_small(const void *w, int w_type, const float *x, int n_in, int n_rows,

@@ -1532,27 +1532,31 @@ __device__ __forceinline__ void gemm_dot(const GFragQ6 &f, const GFragX &x, cons
         acc[i] = q6_block_term(h2f(hd[i][0]), x.dx, (float)isum[i], acc[i]);
 }
 
-// RoPE (ggml mode 0) of one element of a pair in the products' epilogue,
-// with vkv_rope's arithmetic: the angle pos * ts^pair by the running f32
-// product, cos/sin in double rounded to f32, no contraction
-__device__ __forceinline__ float rope_elem(float self, float partner, bool odd, int pair, float pos,
-                                           float ts) {
+// The (cos, sin) pairs of n positions from pos0, [n][head_dim / 2], with
+// vkv_rope's arithmetic: the angle pos * ts^pair by the running f32 product,
+// cos/sin in double rounded to f32.  Evaluated once for all layers of a prompt
+// or an encoder chunk: in every layer's products the double evaluation was
+// ~4 us of a 38-token Q/K/V call's 19 and spilled k_gemm_wide's registers.
+__global__ void __launch_bounds__(256) k_rope_pairs(float2 *tab, int n, int pairs, int64_t pos0, float ts) {
 #pragma clang fp contract(off)
-    float theta = pos;
-    for (int i = 0; i < pair; ++i) theta *= ts;
-    const float c = (float)cos((double)theta), sn = (float)sin((double)theta);
-    return odd ? partner * sn + self * c : self * c - partner * sn;
+    const int i = (int)blockIdx.x * 256 + (int)threadIdx.x;
+    if (i >= n * pairs) return;
+    const int r = i / pairs, p = i - r * pairs;
+    float theta = (float)(pos0 + r);
+    for (int k = 0; k < p; ++k) theta *= ts;
+    tab[i] = make_float2((float)cos((double)theta), (float)sin((double)theta));
 }
 
-// Both elements of a pair at once (one angle): the same bits as rope_elem's
-__device__ __forceinline__ void rope_pair(float &even, float &odd, int pair, float pos, float ts) {
+// RoPE (ggml mode 0) of a pair's element, or of both, in the products'
+// epilogue, without contraction
+__device__ __forceinline__ float rope_elem(float self, float partner, bool odd, float2 cs) {
 #pragma clang fp contract(off)
-    float theta = pos;
-    for (int i = 0; i < pair; ++i) theta *= ts;
-    const float c = (float)cos((double)theta), sn = (float)sin((double)theta);
+    return odd ? partner * cs.y + self * cs.x : self * cs.x - partner * cs.y;
+}
+__device__ __forceinline__ void rope_pair(float &even, float &odd, float2 cs) {
     const float e = even, o = odd;
-    even = e * c - o * sn;
-    odd = e * sn + o * c;
+    even = rope_elem(e, o, false, cs);
+    odd = rope_elem(o, e, true, cs);
 }
 
 // Waves per work group: 8, or 16 when a call has few 16-row tiles (the
@@ -1611,6 +1615,9 @@ __device__ __forceinline__ void gemm_body(const MmArgs &a, const MmOut &o0, cons
                                  : (o0.add ? o0.add : o0.y);
     const int64_t e2i = swiglu ? ot_row : o0.rope ? min(row0 + (ot_r ^ 1), o0.n_rows - 1) : ot_at;
     const float e_2 = e2p[e2i];
+    // the angle's pair (no RoPE: the weights' first bytes, unused)
+    const float2 e_cs = *(o0.rope ? a.rope_tab + (int64_t)ot_col * (a.rope_hd >> 1) + ((ot_row % a.rope_hd) >> 1)
+                                  : reinterpret_cast<const float2 *>(o0.w));
     // the wave's blocks b, b + kw, b + 2 kw, ...: one block's fragments at a
     // time (occupancy, not a second register set, covers the load latency);
     // the first block's (w_first) were requested by the caller
@@ -1663,8 +1670,7 @@ __device__ __forceinline__ void gemm_body(const MmArgs &a, const MmOut &o0, cons
                 float vp = 0.0f;
                 for (int w = 0; w < kw; ++w) vp += red[ct][w][pr][c];
                 if (o0.bias) vp = vp + e_2;
-                y = rope_elem(v0, vp, (orow & 1) != 0, (orow % a.rope_hd) >> 1,
-                              (float)(a.rope_pos0 + ocol), a.rope_ts);
+                y = rope_elem(v0, vp, (orow & 1) != 0, e_cs);
             } else {
                 y = o0.add ? e_2 + v0 : v0;
             }
@@ -2208,7 +2214,8 @@ __device__ __forceinline__ void wide_body(const MmArgs &a, const MmOut &o0, cons
         } else if (o0.rope) {
 #pragma unroll
             for (int i = 0; i < 4; i += 2)
-                rope_pair(y[i], y[i + 1], ((r0 + i) % a.rope_hd) >> 1, (float)(a.rope_pos0 + col), a.rope_ts);
+                rope_pair(y[i], y[i + 1],
+                          a.rope_tab[(int64_t)col * (a.rope_hd >> 1) + (((r0 + i) % a.rope_hd) >> 1)]);
         } else if (o0.add) {
             if (v4 && (reinterpret_cast<uintptr_t>(o0.add) & 15u) == 0) {
                 const float4 r4 = *reinterpret_cast<const float4 *>(o0.add + at);
@@ -2447,6 +2454,11 @@ hipError_t launch_rms_norm_rows(const float *x, int n_rows, int n, const float *
 hipError_t launch_rows_small(const void *w, int w_type, const float *x, int n_in, int n_rows,
                              float *y, hipStream_t st) {
     k_rows_small<<<(unsigned)((n_rows + 3) / 4), 256, 0, st>>>(w, w_type, x, n_in, n_rows, y);
+    return hipGetLastError();
+}
+
+hipError_t launch_rope_pairs(float2 *tab, int n, int pairs, int64_t pos0, float theta_scale, hipStream_t st) {
+    k_rope_pairs<<<(unsigned)((n * (int64_t)pairs + 255) / 256), 256, 0, st>>>(tab, n, pairs, pos0, theta_scale);
     return hipGetLastError();
 }
 
