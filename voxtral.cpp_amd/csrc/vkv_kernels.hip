@@ -1873,6 +1873,61 @@ typedef float float4_t __attribute__((ext_vector_type(4)));
 // group s runs virtual waves [sW, sW + W); it writes its merged (O, M, L)
 // as a partial, which k_window_merge combines in split order.  Only for
 // GQA 1 (a partial per (query row, head, split)).
+// O / L of N dims to an output row (outputs are 16-byte aligned).
+template <int N>
+__device__ __forceinline__ void window_store_out(float *p, const float (&o)[N], float l) {
+    if constexpr (N == 4) {
+        float4 v = make_float4(0, 0, 0, 0);
+        if (l > 0.0f) v = make_float4(o[0] / l, o[1] / l, o[2] / l, o[3] / l);
+        *reinterpret_cast<float4 *>(p) = v;
+    } else {
+        *p = l > 0.0f ? o[0] / l : 0.0f;
+    }
+}
+
+// The W waves of a tile merged in wave order, dims [d, d + N) of its row r
+// (query row rr, kv head g), to the output or the split's partials.  Four
+// dims per thread: at one, each output repeated its row's W exponentials, and
+// a call with few keys per row spent a sixth of its time here (10 F16 tiles
+// of 8 heads, a 38-token prefill: 7.4 -> 6.1 us; 199 tokens over q8_0: 20.8
+// -> 19.1; 16 encoder frames over F32: 9.9 -> 9.4, 128: 30.8 -> 29.6).
+template <int D, int W, int SPL, int N>
+__device__ __forceinline__ void window_merge_waves(const WindowArgs &a, const float (*sm_o)[16][D + N],
+                                                   const float (*sm_m)[16], const float (*sm_l)[16],
+                                                   int r, int d, int rr, int g, int split, int layer) {
+    float M = fmaxf(fmaxf(sm_m[0][r], sm_m[1][r]), fmaxf(sm_m[2][r], sm_m[3][r]));
+#pragma unroll
+    for (int w = 4; w < W; ++w) M = fmaxf(M, sm_m[w][r]);
+    float O[N] = {};
+    float L = 0.0f;
+    if (M != -INFINITY) {
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            const float f = fast_exp2(sm_m[w][r] - M);
+            float o[N];
+            if constexpr (N == 4) *reinterpret_cast<float4 *>(o) = *reinterpret_cast<const float4 *>(&sm_o[w][r][d]);
+            else o[0] = sm_o[w][r][d];
+#pragma unroll
+            for (int e = 0; e < N; ++e) O[e] = fmaf(o[e], f, O[e]);
+            L = fmaf(sm_l[w][r], f, L);
+        }
+    }
+    if constexpr (SPL > 1) {
+        static_assert(N == 4, "whole float4s");
+        const int64_t pv = ((int64_t)(rr - 16 * a.tile0) * a.n_q_heads + g) * SPL + split;
+        *reinterpret_cast<float4 *>(&a.part_o[pv * D + d]) = make_float4(O[0], O[1], O[2], O[3]);
+        if (d == 0) {
+            a.part_ml[pv * 2] = M;
+            a.part_ml[pv * 2 + 1] = L;
+        }
+    } else {
+        const int gqa = a.n_q_heads / a.n_kv_heads;
+        window_store_out<N>(a.out + (int64_t)layer * a.q_lstride +
+                                ((int64_t)(rr / gqa) * a.n_q_heads + g * gqa + rr % gqa) * D + d,
+                            O, L);
+    }
+}
+
 template <int D, int W, int HG = 1, int SPL = 1>
 __global__ void __launch_bounds__(64 * W * HG) k_window_mfma(WindowArgs a) {
     constexpr int KB = D / 16;          // k-blocks of the QK product, d-tiles of PV
@@ -1898,7 +1953,7 @@ __global__ void __launch_bounds__(64 * W * HG) k_window_mfma(WindowArgs a) {
     const uint8_t *vl = a.v + (int64_t)layer * a.layer_bytes;
 
     __shared__ __align__(16) uint8_t sm_v[NWV][16 * VS];   // VS % 8 == 0
-    __shared__ float sm_o[NWV][16][D + 1];
+    __shared__ __align__(16) float sm_o[NWV][16][D + 4];
     __shared__ float sm_m[NWV][16], sm_l[NWV][16];
 
     // ---- Q^T operand: lane holds row lr, dims [DL*lg, DL*lg + DL) as f16 ----
@@ -1928,7 +1983,12 @@ __global__ void __launch_bounds__(64 * W * HG) k_window_mfma(WindowArgs a) {
     const int64_t lo = a.window > 0 ? qa_lo - (a.window - 1) : -((int64_t)1 << 62);
     const int j_lo = (int)max<int64_t>(0, lo - a.key_pos0);
     const int j_hi = (int)min<int64_t>(n_keys, qa_hi - a.key_pos0 + 1);
+    // this lane's row: keys [r_lo, r_lo + r_n), none past the last row (one
+    // 32-bit compare per key instead of four, two of them on 64 bits)
     const int64_t my_lo = a.window > 0 ? q_abs - (a.window - 1) : -((int64_t)1 << 62);
+    const int r_lo = (int)min<int64_t>(n_keys, max<int64_t>(j_lo, my_lo - a.key_pos0));
+    const int r_hi = row_ok ? (int)max<int64_t>(0, min<int64_t>(j_hi, q_abs + 1 - a.key_pos0)) : 0;
+    const uint32_t r_n = (uint32_t)max(0, r_hi - r_lo);
 
     float m = -INFINITY, l = 0.0f;
     float4_t o[KB];
@@ -1978,8 +2038,7 @@ __global__ void __launch_bounds__(64 * W * HG) k_window_mfma(WindowArgs a) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int j = jb + 4 * lg + i;
-            const int64_t kabs = a.key_pos0 + j;
-            const bool ok = row_ok && j >= j_lo && j < j_hi && kabs <= q_abs && kabs >= my_lo;
+            const bool ok = (uint32_t)(j - r_lo) < r_n;
             sc[i] = ok ? st[i] * a.scale_log2 : -INFINITY;
             bm = fmaxf(bm, sc[i]);
         }
@@ -2087,80 +2146,56 @@ __global__ void __launch_bounds__(64 * W * HG) k_window_mfma(WindowArgs a) {
     l += __shfl_xor(l, 32);
     // O^T tile t: lane holds d = 16*t + 4*lg + i of row lr
 #pragma unroll
-    for (int t = 0; t < KB; ++t)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) sm_o[wave][lr][16 * t + 4 * lg + i] = o[t][i];
+    for (int t = 0; t < KB; ++t) *reinterpret_cast<float4_t *>(&sm_o[wave][lr][16 * t + 4 * lg]) = o[t];
     if (lg == 0) {
         sm_m[wave][lr] = m;
         sm_l[wave][lr] = l;
     }
     __syncthreads();
     // head g0 + hh's W waves merge in a fixed order
-    for (int t = threadIdx.x; t < HG * 16 * D; t += 64 * NWV) {
-        const int hh = t / (16 * D);
-        const int r = (t / D) % 16;
-        const int d = t % D;
-        const int rr = tile * 16 + r;
-        if (rr >= n_rows) continue;
-        const int w0 = hh * W;
-        float M = fmaxf(fmaxf(sm_m[w0][r], sm_m[w0 + 1][r]), fmaxf(sm_m[w0 + 2][r], sm_m[w0 + 3][r]));
-#pragma unroll
-        for (int w = 4; w < W; ++w) M = fmaxf(M, sm_m[w0 + w][r]);
-        float O = 0.0f, L = 0.0f;
-        if (M != -INFINITY) {
-#pragma unroll
-            for (int w = 0; w < W; ++w) {
-                const float f = fast_exp2(sm_m[w0 + w][r] - M);
-                O = fmaf(sm_o[w0 + w][r][d], f, O);
-                L = fmaf(sm_l[w0 + w][r], f, L);
-            }
-        }
-        if constexpr (SPL > 1) {
-            const int64_t pv =
-                ((int64_t)(rr - 16 * a.tile0) * a.n_q_heads + g0 + hh) * SPL + split;
-            a.part_o[pv * D + d] = O;
-            if (d == 0) {
-                a.part_ml[pv * 2] = M;
-                a.part_ml[pv * 2 + 1] = L;
-            }
-        } else {
-            const int tk = rr / gqa;
-            float *op = a.out + (int64_t)layer * a.q_lstride +
-                        ((int64_t)tk * a.n_q_heads + (g0 + hh) * gqa + rr % gqa) * D + d;
-            *op = L > 0.0f ? O / L : 0.0f;
-        }
+    for (int t = threadIdx.x; t < HG * 4 * D; t += 64 * NWV) {
+        const int hh = t / (4 * D);
+        const int r = (t / (D / 4)) % 16;
+        if (tile * 16 + r >= n_rows) continue;
+        window_merge_waves<D, W, SPL, 4>(a, &sm_o[hh * W], &sm_m[hh * W], &sm_l[hh * W], r, 4 * (t % (D / 4)),
+                                      tile * 16 + r, g0 + hh, split, layer);
     }
 }
 
 // The split tile's partials of n_vec (query row, head) vectors, merged in
-// split order: one thread per output element.
-template <int SPL>
+// split order: four output dims per thread.
+template <int SPL, int D>
 __global__ void __launch_bounds__(256) k_window_merge(const float *part_o, const float *part_ml,
-                                                      float *out, int64_t n_vec, int D) {
+                                                      float *out, int64_t n_vec) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n_vec * D) return;
-    const int64_t v = i / D;
-    const int d = (int)(i - v * D);
-    float m[SPL], l[SPL], o[SPL];
+    if (i >= n_vec * (D / 4)) return;
+    const int64_t v = i / (D / 4);
+    const int d = 4 * (int)(i % (D / 4));
+    float m[SPL], l[SPL];
+    float4 o[SPL];
 #pragma unroll
     for (int s = 0; s < SPL; ++s) {
         m[s] = part_ml[(v * SPL + s) * 2];
         l[s] = part_ml[(v * SPL + s) * 2 + 1];
-        o[s] = part_o[(v * SPL + s) * D + d];
+        o[s] = *reinterpret_cast<const float4 *>(&part_o[(v * SPL + s) * D + d]);
     }
     float M = m[0];
 #pragma unroll
     for (int s = 1; s < SPL; ++s) M = fmaxf(M, m[s]);
-    float O = 0.0f, L = 0.0f;
+    float O[4] = {};
+    float L = 0.0f;
     if (M != -INFINITY) {
 #pragma unroll
         for (int s = 0; s < SPL; ++s) {
             const float f = fast_exp2(m[s] - M);
-            O = fmaf(o[s], f, O);
+            O[0] = fmaf(o[s].x, f, O[0]);
+            O[1] = fmaf(o[s].y, f, O[1]);
+            O[2] = fmaf(o[s].z, f, O[2]);
+            O[3] = fmaf(o[s].w, f, O[3]);
             L = fmaf(l[s], f, L);
         }
     }
-    out[i] = L > 0.0f ? O / L : 0.0f;
+    window_store_out<4>(out + v * D + d, O, L);
 }
 
 // ---------------------------------------------------------------------------
@@ -2185,7 +2220,7 @@ __global__ void __launch_bounds__(256) k_window_merge(const float *part_o, const
 // (code x fp16 d) on its way into the operand, so every product and sum stays
 // in f32 as on the scalar ALU (k_window, two passes over the keys with a
 // lane per key: a 199-token prefill over 237 keys took 213 us with its append,
-// this 21).  A
+// this 19).  A
 // lane's run of dims is a block (D = 128) or half of one (D = 64).
 
 // A lane's run of DL dims of one K or V row, four at a time as f32.
@@ -2228,6 +2263,12 @@ template <int D, int W, int SPL = 1, bool Q8 = false>
 __device__ __forceinline__ void window_mfma_f32(const WindowArgs &a) {
     constexpr int DL = D / 4;           // contiguous head dims per lane
     constexpr int NT = D / 16;          // 16-dim tiles of P.V
+    // The unsplit head_dim 64 F32 tile (several layers per launch) is at its
+    // 128 VGPRs and 34 KB of LDS: it keeps 64-bit key positions and one output
+    // dim per thread (32 layers of 16 frames: 92.3 us, 93.6 with the others'
+    // form, and with either alone it spills).
+    constexpr bool kLean = SPL == 1 && !Q8 && D == 64;
+    constexpr int NV = kLean ? 1 : 4;   // output dims per thread of the merge
     constexpr int VS = 17;              // LDS stride of the V^T tile (floats)
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -2245,7 +2286,7 @@ __device__ __forceinline__ void window_mfma_f32(const WindowArgs &a) {
     const uint8_t *vl = a.v + (int64_t)layer * a.layer_bytes;
 
     __shared__ float sm_vt[W][D * VS];   // per wave: V^T[d][key]
-    __shared__ float sm_o[W][16][D + 1];
+    __shared__ __align__(16) float sm_o[W][16][D + NV];
     __shared__ float sm_m[W][16], sm_l[W][16];
 
     // ---- Q^T operand: lane holds row lr, dims [DL lg, DL lg + DL) ----
@@ -2274,7 +2315,11 @@ __device__ __forceinline__ void window_mfma_f32(const WindowArgs &a) {
     const int64_t lo = a.window > 0 ? qa_lo - (a.window - 1) : -((int64_t)1 << 62);
     const int j_lo = (int)max<int64_t>(0, lo - a.key_pos0);
     const int j_hi = (int)min<int64_t>(n_keys, qa_hi - a.key_pos0 + 1);
+    // this lane's row: keys [r_lo, r_lo + r_n), none past the last row
     const int64_t my_lo = a.window > 0 ? q_abs - (a.window - 1) : -((int64_t)1 << 62);
+    const int r_lo = (int)min<int64_t>(n_keys, max<int64_t>(j_lo, my_lo - a.key_pos0));
+    const int r_hi = row_ok ? (int)max<int64_t>(0, min<int64_t>(j_hi, q_abs + 1 - a.key_pos0)) : 0;
+    const uint32_t r_n = (uint32_t)max(0, r_hi - r_lo);
 
     float m = -INFINITY, l = 0.0f;
     float4_t o[NT];
@@ -2333,8 +2378,13 @@ __device__ __forceinline__ void window_mfma_f32(const WindowArgs &a) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int j = jb + 4 * lg + i;
-            const int64_t kabs = a.key_pos0 + j;
-            const bool ok = row_ok && j >= j_lo && j < j_hi && kabs <= q_abs && kabs >= my_lo;
+            bool ok;
+            if constexpr (kLean) {
+                const int64_t kabs = a.key_pos0 + j;
+                ok = row_ok && j >= j_lo && j < j_hi && kabs <= q_abs && kabs >= my_lo;
+            } else {
+                ok = (uint32_t)(j - r_lo) < r_n;
+            }
             sc[i] = ok ? st[i] * a.scale_log2 : -INFINITY;
             bm = fmaxf(bm, sc[i]);
         }
@@ -2454,44 +2504,24 @@ __device__ __forceinline__ void window_mfma_f32(const WindowArgs &a) {
     l += __shfl_xor(l, 32);
     // O^T tile T: lane holds d = 16 T + 4 lg + i of row lr
 #pragma unroll
-    for (int T = 0; T < NT; ++T)
+    for (int T = 0; T < NT; ++T) {
+        if constexpr (NV == 4) {
+            *reinterpret_cast<float4_t *>(&sm_o[wave][lr][16 * T + 4 * lg]) = o[T];
+        } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) sm_o[wave][lr][16 * T + 4 * lg + i] = o[T][i];
+            for (int i = 0; i < 4; ++i) sm_o[wave][lr][16 * T + 4 * lg + i] = o[T][i];
+        }
+    }
     if (lg == 0) {
         sm_m[wave][lr] = m;
         sm_l[wave][lr] = l;
     }
     __syncthreads();
-    for (int t = threadIdx.x; t < 16 * D; t += 64 * W) {
-        const int r = t / D;
-        const int d = t % D;
-        const int rr = tile * 16 + r;
-        if (rr >= n_rows) continue;
-        float M = fmaxf(fmaxf(sm_m[0][r], sm_m[1][r]), fmaxf(sm_m[2][r], sm_m[3][r]));
-#pragma unroll
-        for (int w = 4; w < W; ++w) M = fmaxf(M, sm_m[w][r]);
-        float O = 0.0f, L = 0.0f;
-        if (M != -INFINITY) {
-#pragma unroll
-            for (int w = 0; w < W; ++w) {
-                const float f = fast_exp2(sm_m[w][r] - M);
-                O = fmaf(sm_o[w][r][d], f, O);
-                L = fmaf(sm_l[w][r], f, L);
-            }
-        }
-        if constexpr (SPL > 1) {
-            const int64_t pv = ((int64_t)(rr - 16 * a.tile0) * a.n_q_heads + g) * SPL + split;
-            a.part_o[pv * D + d] = O;
-            if (d == 0) {
-                a.part_ml[pv * 2] = M;
-                a.part_ml[pv * 2 + 1] = L;
-            }
-        } else {
-            const int tk = rr / gqa;
-            float *op = a.out + (int64_t)layer * a.q_lstride +
-                        ((int64_t)tk * a.n_q_heads + g * gqa + rr % gqa) * D + d;
-            *op = L > 0.0f ? O / L : 0.0f;
-        }
+    for (int t = threadIdx.x; t < 16 * D / NV; t += 64 * W) {
+        const int r = t / (D / NV);
+        if (tile * 16 + r >= n_rows) continue;
+        window_merge_waves<D, W, SPL, NV>(a, sm_o, sm_m, sm_l, r, NV * (t % (D / NV)), tile * 16 + r, g,
+                                          split, layer);
     }
 }
 
@@ -2780,10 +2810,10 @@ hipError_t launch_window(int dtype, bool valu, const WindowArgs &a_in, hipStream
                 else
                     hipLaunchKernelGGL((k_window_mfma<64, 4, 1, kWinSplit>), gs, dim3(256), 0, st, b);
                 const int64_t n_vec = (int64_t)std::min(16 * nt, n_rows - 16 * t0) * a.n_q_heads;
-                hipLaunchKernelGGL(k_window_merge<kWinSplit>,
-                                   dim3((unsigned)((n_vec * 64 + 255) / 256)), dim3(256), 0, st,
+                hipLaunchKernelGGL((k_window_merge<kWinSplit, 64>),
+                                   dim3((unsigned)((n_vec * 16 + 255) / 256)), dim3(256), 0, st,
                                    (const float *)a.part_o, (const float *)a.part_ml,
-                                   a.out + (int64_t)16 * t0 * a.n_q_heads * 64, n_vec, 64);
+                                   a.out + (int64_t)16 * t0 * a.n_q_heads * 64, n_vec);
             }
         } else if (dtype == VKV_DTYPE_F32) {
             // (8 waves for the per-layer calls, as the F16 tile takes, measured
