@@ -328,3 +328,49 @@ def test_q8_0_embedding_row():
                   hip_stream=stream_ptr())
         want = oracle.dequantize(oracle.Q8_0, table[token * rb:(token + 1) * rb], dim) + audio
         np.testing.assert_array_equal(host(y), want)
+
+
+def calls_of(mats, n_in, x, nw, ws, epilogue=vkv.MV_STORE):
+    """one vkv.matvec call: mats' (dtype, rows) in order; their outputs"""
+    ys = [torch.full((n,), np.nan, dtype=torch.float32, device=dev()) for _, n in mats]
+    vkv.matvec(x.data_ptr(), n_in,
+               [(w.data_ptr(), dt, n, y.data_ptr()) for w, (dt, n), y in zip(ws, mats, ys)],
+               norm_w_ptr=nw.data_ptr() if nw is not None else None, eps=EPS, epilogue=epilogue,
+               hip_stream=stream_ptr())
+    return ys
+
+
+# 1, 2 and 3 steps per row; rows that a wave requests at once and that it
+# streams (from 1, 2 or 4 per wave on, by type and width); the largest input
+@pytest.mark.parametrize("n_in,n_rows", [(512, 13), (3072, 3071), (4096, 9216), (5120, 1021), (5120, 2500),
+                                         (8192, 5000), (12288, 777), (9216, 3072)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_a_matrix_gives_the_same_bits_in_every_kind_of_call(n_in, n_rows, norm):
+    """Calls of one format, of both K-quants, and of any mix run kernels of
+    their own: each matrix's rows are the same alone and in any of them.  A
+    SwiGLU pair and a GELU product are the functions of the plain products."""
+    rng = np.random.default_rng(n_in + n_rows + norm)
+    x, nw, _ = inputs(rng, n_in)
+    x, nw = to_dev(x * 0.2), to_dev(nw) if norm else None
+    types = [vkv.Q4_K, vkv.Q6_K, vkv.Q8_0]
+    w = {t: to_dev(random_matrix(rng, t, n_rows, n_in, 0.02)) for t in types}
+    w2 = {t: to_dev(random_matrix(rng, t, n_rows, n_in, 0.02)) for t in types}
+    alone = {t: calls_of([(t, n_rows)], n_in, x, nw, [w[t]])[0] for t in types}
+    other = {t: calls_of([(t, n_rows)], n_in, x, nw, [w2[t]])[0] for t in types}
+    for mix in ([vkv.Q4_K, vkv.Q6_K], [vkv.Q6_K, vkv.Q8_0], [vkv.Q8_0, vkv.Q4_K, vkv.Q6_K]):
+        got = calls_of([(t, n_rows) for t in mix], n_in, x, nw, [w[t] for t in mix])
+        for t, y in zip(mix, got):
+            assert torch.equal(y, alone[t]), (mix, t)
+    for t in types:
+        assert torch.isfinite(alone[t]).all()
+        g, u = alone[t].double(), other[t].double()
+        gelu = calls_of([(t, n_rows)], n_in, x, nw, [w[t]], vkv.MV_GELU)[0].double()
+        want = 0.5 * g * (1 + torch.erf(g / 2 ** 0.5))
+        # a few f32 roundings; erf's cancellation at the negative end scales with |g|
+        assert ((gelu - want).abs() <= 1e-6 * g.abs() + 1e-30).all()
+        y = torch.full((n_rows,), np.nan, dtype=torch.float32, device=dev())
+        vkv.matvec(x.data_ptr(), n_in, [(w[t].data_ptr(), t, n_rows, y.data_ptr()), (w2[t].data_ptr(), t, n_rows, None)],
+                   norm_w_ptr=nw.data_ptr() if norm else None, eps=EPS, epilogue=vkv.MV_SWIGLU,
+                   hip_stream=stream_ptr())
+        want = g / (1 + torch.exp(-g)) * u
+        assert ((y.double() - want).abs() <= 1e-6 * want.abs() + 1e-30).all()

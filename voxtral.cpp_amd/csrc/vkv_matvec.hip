@@ -46,8 +46,11 @@ constexpr int kQ6Bytes = 210;
 constexpr int kQ8Bytes = 34;                   // one block_q8_0: fp16 d, 32 int8
 constexpr int kQ8Per256 = 8 * kQ8Bytes;        // bytes of 256 Q8_0 weights
 
-// the weight format a work group streams (one per work group)
-enum WKind { kWQ4 = 0, kWQ6 = 1, kWQ8 = 2 };
+// The weight format a work group streams.  As a k_matvec parameter also those
+// of a call: kWK, Q4_K beside Q6_K matrices; kWAny, any mix (and GELU).
+enum WKind { kWQ4 = 0, kWQ6 = 1, kWQ8 = 2, kWK = 3, kWAny = 4 };
+// SwiGLU: never, always, as the call says
+enum Pair { kNoPair = 0, kPair = 1, kPairAny = 2 };
 constexpr uint32_t kOob = 0xFFFFFF00u;   // buffer offset past every resource: loads read 0
 
 // Q8_K image of the input vector, per work group (q8_0 image for Q8_0 rows:
@@ -634,12 +637,18 @@ __device__ __forceinline__ void argmax_publish(const MvArgs &a, unsigned long lo
 // WK (the work group's weight format) is a template parameter so that every
 // load writes its final registers (a load feeding a merge of two paths would
 // be copied, and the copy waits for the load).  Q8_0 rows keep D6 units in
-// flight (17 dwords a task against Q6_K's 19).
-template <int S, int D4, int D6, bool ONE, int WK, bool AMAX, bool NE>
+// flight (17 dwords a task against Q6_K's 19).  NORM, PAIR and GELU: what of
+// the input's norm, SwiGLU and GELU the call may take (the code's size counts,
+// see k_matvec).
+template <int S, int D4, int D6, bool ONE, int WK, bool AMAX, bool NORM, int PAIR, bool GELU>
 __device__ __forceinline__ void matvec_body(const MvArgs &a, const MvOut &o0, const MvOut &ob,
                                             int row0, int nrow, ActSmem &sm) {
     const int lane = threadIdx.x & 63;
-    const bool swiglu = a.swiglu != 0;
+    const bool swiglu = PAIR == kPairAny ? a.swiglu != 0 : PAIR == kPair;
+    // With a norm, the inputs of up to 4096 (S == 1) request its weights (and
+    // the ada row) together with x, so that the norm costs one round trip.
+    constexpr bool NE = NORM && S == 1;
+    const float *nw = NORM ? a.norm_w : nullptr, *ada = NORM ? a.ada : nullptr;
     const int mats = swiglu ? 2 : 1;
     const int units = nrow * S * mats;
     const int nb = a.n_in >> 8, tasks = 4 * nb;
@@ -651,7 +660,7 @@ __device__ __forceinline__ void matvec_body(const MvArgs &a, const MvOut &o0, co
     constexpr int D = WK == kWQ4 ? D4 : D6;   // units in flight per dtype
     constexpr int NBW = S == 1 ? 4 : 4 * S;   // n_in <= 4096 / 12288
     ActRegs<NBW, NE> ar;
-    act_load(ar, a.x, a.n_in, a.norm_w, a.ada);
+    act_load(ar, a.x, a.n_in, nw, ada);
     using Frag = std::conditional_t<WK == kWQ4, FragQ4, std::conditional_t<WK == kWQ8, FragQ8, FragQ6>>;
     // Every weight load is unconditional (units past the end read zeros):
     // a load issued on one path only makes the compiler's wait counts assume
@@ -672,7 +681,7 @@ __device__ __forceinline__ void matvec_body(const MvArgs &a, const MvOut &o0, co
     const float *ap = o0.add ? o0.add : o0.y;
     const float addv = ap[min(row0 + min(lane, max(nrow - 1, 0)), o0.n_rows - 1)];
     __builtin_amdgcn_sched_barrier(0);
-    act_finish<NBW, NE, false, WK == kWQ8>(ar, a.n_in, a.norm_w, a.ada, a.eps, sm, nullptr);
+    act_finish<NBW, NE, false, WK == kWQ8>(ar, a.n_in, nw, ada, a.eps, sm, nullptr);
 
     const XFrag xr = xfrag<WK>(sm, min(lane, tasks - 1));   // the only step when S == 1
 
@@ -701,7 +710,7 @@ __device__ __forceinline__ void matvec_body(const MvArgs &a, const MvOut &o0, co
             if (!swiglu) {
                 const float res = __builtin_bit_cast(
                     float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, addv), u / (S * mats)));
-                const float yv = a.gelu ? gelu_erf(r) : o0.add ? res + r : r;
+                const float yv = GELU && a.gelu ? gelu_erf(r) : o0.add ? res + r : r;
                 if (lane == 0) o0.y[row] = yv;
                 if constexpr (AMAX) {
                     const uint32_t b = __builtin_bit_cast(uint32_t, yv);
@@ -741,7 +750,16 @@ __device__ __forceinline__ void matvec_body(const MvArgs &a, const MvOut &o0, co
 // D4 / D6: a wave's units in flight for Q4_K / Q6_K (and Q8_0) rows; ONE: every wave's
 // units fit (the launch picks it from the units per wave, so that a decoder
 // product's wave requests all its weights at once and streams nothing).
-template <int S, int D4, int D6, bool ONE, bool AMAX>
+//
+// WK, NORM, PAIR: the call's weight formats and epilogue.  A decoder token
+// cycles through its layer's kernels, about 160 launches of 3 to 12 us, and two
+// CUs share 64 KB of instruction cache, so a layer's code has to stay in it:
+// with every format and epilogue in each kernel (the four products' kernels
+// 117 KB, their bodies up to 12.7 KB) the token took 1.34 to 1.40 ms according
+// to where the linker put them, a period of 8 KB.  With only what a call takes
+// (30 KB for the Q4_K / Q6_K file's four, beside 15 KB of attention) it takes
+// 1.26 to 1.28 ms at every placement, a Q8_0 token 1.22 (1.28 to 1.31 before).
+template <int S, int D4, int D6, bool ONE, bool AMAX, int WK, bool NORM, int PAIR>
 __global__ void __launch_bounds__(256) k_matvec(MvArgs a) {
     __shared__ ActSmem sm;
     // wave-uniform (readfirstlane): the row range and the unit loop follow
@@ -752,20 +770,17 @@ __global__ void __launch_bounds__(256) k_matvec(MvArgs a) {
     for (int k = 1; k < kMvMaxOuts; ++k)
         if (k < a.n_outs && (int)blockIdx.x >= a.out[k].wg0) seg = k;
     const MvOut o0 = out_at(a, seg);
-    const MvOut ob = a.swiglu ? a.out[1] : o0;
+    const MvOut ob = (PAIR == kPairAny ? a.swiglu != 0 : PAIR == kPair) ? a.out[1] : o0;
     const int row0 = ((int)blockIdx.x - o0.wg0) * a.rows_per_wg + wave * (a.rows_per_wg >> 2);
     const int nrow = max(0, min(a.rows_per_wg >> 2, o0.n_rows - row0));
-    // With a norm (S == 1: the inputs of up to 4096), its weights (and the ada
-    // row) are requested together with x, so the norm costs one round trip.
-    if (S == 1 && a.norm_w) {
-        if (o0.dtype == VKV_DTYPE_Q4_K) matvec_body<S, D4, D6, ONE, kWQ4, AMAX, true>(a, o0, ob, row0, nrow, sm);
-        else if (o0.dtype == VKV_DTYPE_Q8_0) matvec_body<S, D4, D6, ONE, kWQ8, AMAX, true>(a, o0, ob, row0, nrow, sm);
-        else matvec_body<S, D4, D6, ONE, kWQ6, AMAX, true>(a, o0, ob, row0, nrow, sm);
-    } else {
-        if (o0.dtype == VKV_DTYPE_Q4_K) matvec_body<S, D4, D6, ONE, kWQ4, AMAX, false>(a, o0, ob, row0, nrow, sm);
-        else if (o0.dtype == VKV_DTYPE_Q8_0) matvec_body<S, D4, D6, ONE, kWQ8, AMAX, false>(a, o0, ob, row0, nrow, sm);
-        else matvec_body<S, D4, D6, ONE, kWQ6, AMAX, false>(a, o0, ob, row0, nrow, sm);
-    }
+    auto body = [&](auto wk) __attribute__((always_inline)) {
+        matvec_body<S, D4, D6, ONE, decltype(wk)::value, AMAX, NORM, PAIR, WK == kWAny>(a, o0, ob, row0,
+                                                                                        nrow, sm);
+    };
+    if constexpr (WK < kWK) body(std::integral_constant<int, WK>{});
+    else if (o0.dtype == VKV_DTYPE_Q4_K) body(std::integral_constant<int, kWQ4>{});
+    else if (WK == kWAny && o0.dtype == VKV_DTYPE_Q8_0) body(std::integral_constant<int, kWQ8>{});
+    else body(std::integral_constant<int, kWQ6>{});
 }
 
 __global__ void __launch_bounds__(256) k_q8k_quant(const float *x, int n, const float *nw,
@@ -2255,6 +2270,40 @@ __global__ void __launch_bounds__(64 * RT * (SW ? 2 : 1), wide_pre(CT, RT) == 1 
     else wide_body<kWQ6, CT, RT, SW>(a, o0, o1, sm);
 }
 
+// k_matvec for the call's weight formats, norm and epilogue (a fused argmax has
+// one matrix and neither SwiGLU nor GELU)
+template <int S, int D4, int D6, bool ONE, bool AMAX>
+void launch_mv(const MvArgs &a, int n_wg, hipStream_t st) {
+    using std::integral_constant;
+    const int t = a.out[0].dtype;
+    bool same = true, q80 = t == VKV_DTYPE_Q8_0;
+    for (int k = 1; k < a.n_outs; ++k) {
+        same = same && a.out[k].dtype == t;
+        q80 = q80 || a.out[k].dtype == VKV_DTYPE_Q8_0;
+    }
+    auto go = [&](auto wk, auto norm, auto pair) {
+        k_matvec<S, D4, D6, ONE, AMAX, decltype(wk)::value, decltype(norm)::value, decltype(pair)::value>
+            <<<n_wg, 256, 0, st>>>(a);
+    };
+    auto one_format = [&](auto norm, auto pair) {
+        if (t == VKV_DTYPE_Q4_K) go(integral_constant<int, kWQ4>{}, norm, pair);
+        else if (t == VKV_DTYPE_Q6_K) go(integral_constant<int, kWQ6>{}, norm, pair);
+        else go(integral_constant<int, kWQ8>{}, norm, pair);
+    };
+    auto formats = [&](auto norm) {
+        const integral_constant<int, kNoPair> none;
+        if constexpr (!AMAX) {
+            if (a.gelu || (!same && q80))
+                return go(integral_constant<int, kWAny>{}, norm, integral_constant<int, kPairAny>{});
+            if (!same) return go(integral_constant<int, kWK>{}, norm, none);
+            if (a.swiglu) return one_format(norm, integral_constant<int, kPair>{});
+        }
+        one_format(norm, none);
+    };
+    if (a.norm_w) formats(std::true_type{});
+    else formats(std::false_type{});
+}
+
 }  // namespace
 
 hipError_t launch_matvec(const MvArgs &a, int n_wg, hipStream_t st) {
@@ -2273,15 +2322,15 @@ hipError_t launch_matvec(const MvArgs &a, int n_wg, hipStream_t st) {
     for (int k = 0; k < a.n_outs; ++k) (a.out[k].dtype == VKV_DTYPE_Q4_K ? q4 : q6) = true;
     auto fits = [&](int d4, int d6) { return (!q4 || units <= d4) && (!q6 || units <= d6); };
     const bool one = fits(6, 3);
-    if (a.amax) k_matvec<1, 3, 4, false, true><<<n_wg, 256, 0, st>>>(a);
-    else if (S == 1 && fits(3, 2)) k_matvec<1, 3, 2, true, false><<<n_wg, 256, 0, st>>>(a);
-    else if (S == 1 && one) k_matvec<1, 6, 3, true, false><<<n_wg, 256, 0, st>>>(a);
-    else if (S == 1) k_matvec<1, 4, 4, false, false><<<n_wg, 256, 0, st>>>(a);
-    else if (S == 2 && fits(2, 2)) k_matvec<2, 2, 2, true, false><<<n_wg, 256, 0, st>>>(a);
-    else if (S == 2 && one) k_matvec<2, 6, 3, true, false><<<n_wg, 256, 0, st>>>(a);
-    else if (S == 2) k_matvec<2, 2, 2, false, false><<<n_wg, 256, 0, st>>>(a);
-    else if (one) k_matvec<3, 6, 3, true, false><<<n_wg, 256, 0, st>>>(a);
-    else k_matvec<3, 2, 2, false, false><<<n_wg, 256, 0, st>>>(a);
+    if (a.amax) launch_mv<1, 3, 4, false, true>(a, n_wg, st);
+    else if (S == 1 && fits(3, 2)) launch_mv<1, 3, 2, true, false>(a, n_wg, st);
+    else if (S == 1 && one) launch_mv<1, 6, 3, true, false>(a, n_wg, st);
+    else if (S == 1) launch_mv<1, 4, 4, false, false>(a, n_wg, st);
+    else if (S == 2 && fits(2, 2)) launch_mv<2, 2, 2, true, false>(a, n_wg, st);
+    else if (S == 2 && one) launch_mv<2, 6, 3, true, false>(a, n_wg, st);
+    else if (S == 2) launch_mv<2, 2, 2, false, false>(a, n_wg, st);
+    else if (one) launch_mv<3, 6, 3, true, false>(a, n_wg, st);
+    else launch_mv<3, 2, 2, false, false>(a, n_wg, st);
     return hipGetLastError();
 }
 
