@@ -1,10 +1,11 @@
-"""A decoder layer's kernels stay in the instruction cache.
+"""A layer's kernels stay in the instruction cache.
 
-Two CUs share 64 KB of it, and a token cycles through its layer's kernels at 3
-to 12 us a launch: when their code did not fit, the token's time changed by 4%
-with where the linker had put them.  The kernels that a layer launches (the
-widths of the 4B decoder, whose launch shapes launch_matvec picks) may take
-three quarters of it, whatever else is built."""
+Two CUs share 64 KB of it, and a decoder token or a 4-frame encoder chunk
+cycles through its layer's kernels at 3 to 12 us a launch: when their code did
+not fit, the times changed by 2 to 4% with where the linker had put them.  The
+kernels that a layer launches (at the 4B model's widths, whose launch shapes
+launch_matvec and launch_gemm_kq pick) may take three quarters of it, whatever
+else is built."""
 import os
 import re
 import struct
@@ -14,7 +15,6 @@ import pytest
 import vkv
 
 ICACHE = 64 * 1024
-ATTENTION = [r"k_decodeI\w*FmtF16\w*ELi4ELb1ELi4ELi2E", r"9k_combineE"]
 
 
 def code_objects(path):
@@ -53,27 +53,39 @@ def kernel_sizes(path):
     return out
 
 
+def args(v):
+    return "".join(f"L{'b' if isinstance(x, bool) else 'i'}{int(x)}E" for x in v)
+
+
 def matvec(shape, kind):
-    """k_matvec<S, D4, D6, ONE, false, kind...>, or the shape's only kernel"""
-    def args(v):
-        return "".join(f"L{'b' if isinstance(x, bool) else 'i'}{int(x)}E" for x in v)
+    """k_matvec<steps, units in flight (2), all at once, no argmax, formats, norm, SwiGLU>"""
     return f"k_matvecI{args(shape + (False,))}({args(kind)})?EEv"
 
 
-# (steps, units in flight, all at once), (formats, norm, SwiGLU): Q/K/V, O, W1/W3, W2
+def gemm(waves, fmt, epilogue):
+    """k_gemm_kq<waves, one column tile, input quantized inside, formats, epilogue>"""
+    return f"k_gemm_kqI{args((waves, 1, True))}({args((fmt, epilogue))})?EEv"
+
+
+DECODE = [r"k_decodeI\w*FmtF16\w*ELi4ELb1ELi4ELi2E", r"9k_combineE"]
+WINDOW = [r"\d\dk_window_mfma_f32_64_splitE", r"k_window_mergeI"]
+# Q/K/V, O, W1/W3, W2 and the attention
 LAYERS = {
-    "Q4_K and Q6_K": [((1, 3, 2, True), (3, True, 0)), ((1, 3, 2, True), (0, False, 0)),
-                      ((1, 4, 4, False), (0, True, 1)), ((3, 2, 2, False), (1, False, 0))],
-    "Q8_0": [((1, 3, 2, True), (2, True, 0)), ((1, 6, 3, True), (2, False, 0)),
-             ((1, 4, 4, False), (2, True, 1)), ((3, 2, 2, False), (2, False, 0))],
+    "decoder, Q4_K and Q6_K": [matvec((1, 3, 2, True), (3, True, 0)), matvec((1, 3, 2, True), (0, False, 0)),
+                               matvec((1, 4, 4, False), (0, True, 1)), matvec((3, 2, 2, False), (1, False, 0)),
+                               *DECODE],
+    "decoder, Q8_0": [matvec((1, 3, 2, True), (2, True, 0)), matvec((1, 6, 3, True), (2, False, 0)),
+                      matvec((1, 4, 4, False), (2, True, 1)), matvec((3, 2, 2, False), (2, False, 0)), *DECODE],
+    # (O and W2 in one kernel)
+    "encoder chunk, Q8_0": [gemm(8, 2, 0), gemm(16, 2, 0), gemm(8, 2, 1), *WINDOW],
 }
 
 
-@pytest.mark.parametrize("formats", LAYERS)
-def test_a_decoder_layers_kernels_fit_the_instruction_cache(formats):
+@pytest.mark.parametrize("layer", LAYERS)
+def test_a_layers_kernels_fit_the_instruction_cache(layer):
     sizes = kernel_sizes(os.path.join(os.path.dirname(vkv.__file__), "libvkv.so"))
     found = {}
-    for pattern in [matvec(*k) for k in LAYERS[formats]] + ATTENTION:
+    for pattern in LAYERS[layer]:
         hits = {n: s for n, s in sizes.items() if re.search(pattern, n)}
         assert len(hits) == 1, (pattern, sorted(hits))
         found.update(hits)

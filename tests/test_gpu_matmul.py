@@ -348,3 +348,47 @@ def test_q8_0_matches_the_single_row_kernel_and_rejects_mixing():
         vkv.matmul(xd.data_ptr(), 1, n_in, [(wd.data_ptr(), vkv.Q8_0, n_rows, y2.data_ptr()),
                                             (wd.data_ptr(), vkv.Q4_K, 16, y1.data_ptr())],
                    ws_ptr, ws_b, hip_stream=stream_ptr())
+
+
+@pytest.mark.parametrize("P", [3, 11, 24])   # quantized inside; one column tile; two
+@pytest.mark.parametrize("n_in,n_rows", [(1280, 500), (1280, 2100), (3072, 2063)])   # 16 and 8 waves
+@pytest.mark.parametrize("norm", [False, True])
+def test_a_matrix_gives_the_same_rows_in_every_kind_of_call(P, n_in, n_rows, norm):
+    """Calls of one format and of both K-quants, and each epilogue, run kernels
+    of their own: a matrix's rows are the same bits alone and beside another
+    format's; SwiGLU (its waves split K in halves: the f32 order of the sums,
+    1e-5 x sum |w||x|) and GELU are the functions of the plain products."""
+    rng = np.random.default_rng(P + n_in + n_rows + norm)
+    x = torch.from_numpy(rng.standard_normal((P, n_in)).astype(np.float32)).to(dev()) * 0.5
+    nw = torch.from_numpy(rng.uniform(0.5, 1.5, n_in).astype(np.float32)).to(dev())
+    t, wp, wb = workspace(P, n_in)
+
+    def call(mats, epilogue=vkv.MV_STORE):
+        ys = [torch.full((P, n_rows), np.nan, device=dev()) for _ in mats]
+        vkv.matmul(x.data_ptr(), P, n_in, [(w.data_ptr(), dt, n_rows, y.data_ptr()) for (dt, w), y in zip(mats, ys)],
+                   wp, wb, norm_w_ptr=nw.data_ptr() if norm else None, eps=EPS, epilogue=epilogue,
+                   hip_stream=stream_ptr())
+        return ys
+
+    types = [vkv.Q4_K, vkv.Q6_K, vkv.Q8_0]
+    w = {dt: [to_dev(random_matrix(rng, dt, n_rows, n_in, 0.02)) for _ in range(2)] for dt in types}
+    alone = {dt: [call([(dt, m)])[0] for m in w[dt]] for dt in types}
+    for mix in ([vkv.Q4_K, vkv.Q6_K], [vkv.Q6_K, vkv.Q4_K], [vkv.Q8_0, vkv.Q8_0]):
+        for dt, y in zip(mix, call([(dt, w[dt][0]) for dt in mix])):
+            assert torch.equal(y, alone[dt][0])
+    h = x * torch.rsqrt((x * x).mean(1, keepdim=True) + EPS) * nw if norm else x
+    for dt in types:
+        g, u = (y.double() for y in alone[dt])
+        assert torch.isfinite(g).all()
+        gelu = call([(dt, w[dt][0])], vkv.MV_GELU)[0].double()
+        want = 0.5 * g * (1 + torch.erf(g / 2 ** 0.5))
+        assert ((gelu - want).abs() <= 1e-6 * g.abs() + 1e-30).all()
+        mags = []
+        for m in w[dt]:
+            f = torch.empty(n_rows, n_in, device=dev())
+            vkv.dequantize(dt, m.data_ptr(), n_rows * n_in, f.data_ptr(), hip_stream=stream_ptr())
+            mags.append((h.abs() @ f.abs().T).double() * 1.05)   # (x's own codes: within 5%)
+        y = call([(dt, m) for m in w[dt]], vkv.MV_SWIGLU)[0].double()
+        sg = g / (1 + torch.exp(-g))
+        bound = REL * (1.1 * mags[0] * u.abs() + sg.abs() * mags[1]) + 1e-6 * (sg * u).abs()
+        assert ((y - sg * u).abs() <= bound + 1e-30).all()

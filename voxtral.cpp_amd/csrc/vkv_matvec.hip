@@ -51,6 +51,8 @@ constexpr int kQ8Per256 = 8 * kQ8Bytes;        // bytes of 256 Q8_0 weights
 enum WKind { kWQ4 = 0, kWQ6 = 1, kWQ8 = 2, kWK = 3, kWAny = 4 };
 // SwiGLU: never, always, as the call says
 enum Pair { kNoPair = 0, kPair = 1, kPairAny = 2 };
+// k_gemm_kq's epilogues: stored, with a residual or RoPE; SwiGLU; GELU
+enum MmEpilogue { kMmPlain = 0, kMmPair = 1, kMmGelu = 2 };
 constexpr uint32_t kOob = 0xFFFFFF00u;   // buffer offset past every resource: loads read 0
 
 // Q8_K image of the input vector, per work group (q8_0 image for Q8_0 rows:
@@ -1580,7 +1582,7 @@ __device__ __forceinline__ void rope_pair(float &even, float &odd, float2 cs) {
 // input rows each) per work group: a wave loads each weight block once and
 // applies it to every column tile, so the weights are read once per 16 CT
 // input rows.
-template <int WK, int W, int CT, bool ALLH, class GF>
+template <int WK, int W, int CT, bool ALLH, int EPI, class GF>
 __device__ __forceinline__ void gemm_body(const MmArgs &a, const MmOut &o0, const MmOut &o1,
                                           uint32_t (*hdr)[16][6], float (*red)[W][16][17],
                                           const XImage &im, const GF &w_first) {
@@ -1589,7 +1591,7 @@ __device__ __forceinline__ void gemm_body(const MmArgs &a, const MmOut &o0, cons
     // the descriptor's values)
     const int lane = threadIdx.x & 63, kg = lane >> 4, rr = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const bool swiglu = a.swiglu != 0;
+    constexpr bool swiglu = EPI == kMmPair;
     const int nb = a.n_in >> 8;
     const uint32_t bbytes = WK == kWQ4 ? kQ4Bytes : WK == kWQ8 ? kQ8Per256 : kQ6Bytes;
     const uint32_t rbytes = (uint32_t)nb * bbytes;
@@ -1677,7 +1679,7 @@ __device__ __forceinline__ void gemm_body(const MmArgs &a, const MmOut &o0, cons
                 for (int w = 0; w < kw; ++w) v1 += red[ct][kw + w][r][c];
                 if (o1.bias) v1 = v1 + e_2;
                 y = silu(v0) * v1;
-            } else if (a.gelu) {
+            } else if (EPI == kMmGelu) {
                 y = gelu_erf(v0);
             } else if (o0.rope) {
                 // the pair's other row is in this tile: its sum and bias
@@ -1694,6 +1696,12 @@ __device__ __forceinline__ void gemm_body(const MmArgs &a, const MmOut &o0, cons
     }
 }
 
+// FMT, EPI: the call's weight formats (kWK: both K-quants) and epilogue, each
+// kernel with only those, for the instruction cache (see k_matvec).  The
+// 4-frame encoder chunk's kernels were 102 KB with all three formats and
+// epilogues in each and it took 1.667 or 1.699 ms on a Q8_0 file as they moved,
+// 1.59 on a K-quant one; with their own, 47 KB (Q8_0), it takes 1.60 and 1.52.
+//
 // (the body is in the kernel itself: a reference to the by-value kernel
 // argument passed through one more inlined function made the compiler copy
 // the argument to scratch memory)
@@ -1706,7 +1714,7 @@ __host__ __device__ constexpr size_t fused_lds_bytes(int cols, int n_in, bool no
            (norm ? (size_t)3 * n_in * 4 : 0);
 }
 
-template <int W, int CT, bool FQ>
+template <int W, int CT, bool FQ, int FMT, int EPI>
 __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) k_gemm_kq(MmArgs a) {
     __shared__ uint32_t hdr[W][16][6];
     __shared__ float red[CT][W][16][17];
@@ -1715,7 +1723,8 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))
     for (int k = 1; k < kMvMaxOuts; ++k)
         if (k < a.n_outs && (int)blockIdx.x >= a.out[k].tile0) seg = k;
     const MmOut o0 = mm_out_at(a, seg);
-    const MmOut o1 = a.swiglu ? a.out[1] : o0;
+    constexpr bool swiglu = EPI == kMmPair;
+    const MmOut o1 = swiglu ? a.out[1] : o0;
     // one weight dtype per work group (both SwiGLU matrices share it)
     auto run = [&](auto wk) __attribute__((always_inline)) {
         constexpr int WK = decltype(wk)::value;
@@ -1729,8 +1738,8 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))
         const uint32_t bbytes = WK == kWQ4 ? kQ4Bytes : WK == kWQ8 ? kQ8Per256 : kQ6Bytes;
         const uint32_t rbytes = (uint32_t)nb * bbytes;
         const int row = min(((int)blockIdx.x - o0.tile0) * 16 + rr, o0.n_rows - 1);
-        const int kw = a.swiglu ? W / 2 : W;
-        const int m = a.swiglu ? wave / kw : 0, wm = wave - m * kw;
+        const int kw = swiglu ? W / 2 : W;
+        const int m = swiglu ? wave / kw : 0, wm = wave - m * kw;
         const __amdgpu_buffer_rsrc_t rs0 = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<uint8_t *>(o0.w), (short)0, (int)(rbytes * (uint32_t)o0.n_rows), 0x00020000);
         const __amdgpu_buffer_rsrc_t rs1 = __builtin_amdgcn_make_buffer_rsrc(
@@ -1777,10 +1786,10 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))
         } else {
             pre();
         }
-        gemm_body<WK, W, CT, FQ>(a, o0, o1, hdr, red, im, wf);
+        gemm_body<WK, W, CT, FQ, EPI>(a, o0, o1, hdr, red, im, wf);
     };
-    if (o0.dtype == VKV_DTYPE_Q4_K) run(std::integral_constant<int, kWQ4>{});
-    else if (o0.dtype == VKV_DTYPE_Q8_0) run(std::integral_constant<int, kWQ8>{});
+    if constexpr (FMT < kWK) run(std::integral_constant<int, FMT>{});
+    else if (o0.dtype == VKV_DTYPE_Q4_K) run(std::integral_constant<int, kWQ4>{});
     else run(std::integral_constant<int, kWQ6>{});
 }
 
@@ -2403,6 +2412,32 @@ hipError_t launch_gemm_wide(MmArgs a, hipStream_t st) {
 }
 }  // namespace
 
+namespace {
+// k_gemm_kq for the call's weight formats and epilogue
+template <int W, int CT, bool FQ>
+void launch_kq(const MmArgs &a, dim3 g, size_t lds, hipStream_t st) {
+    using std::integral_constant;
+    const int t = a.out[0].dtype;
+    bool same = true;
+    for (int k = 1; k < a.n_outs; ++k) same = same && a.out[k].dtype == t;
+    auto go = [&](auto fmt, auto epi) {
+        k_gemm_kq<W, CT, FQ, decltype(fmt)::value, decltype(epi)::value><<<g, 64 * W, lds, st>>>(a);
+    };
+    auto formats = [&](auto epi) {
+        // (a SwiGLU pair is of one format)
+        if (t == VKV_DTYPE_Q8_0) return go(integral_constant<int, kWQ8>{}, epi);
+        if constexpr (decltype(epi)::value != kMmPair) {
+            if (!same) return go(integral_constant<int, kWK>{}, epi);
+        }
+        if (t == VKV_DTYPE_Q4_K) go(integral_constant<int, kWQ4>{}, epi);
+        else go(integral_constant<int, kWQ6>{}, epi);
+    };
+    if (a.swiglu) formats(integral_constant<int, kMmPair>{});
+    else if (a.gelu) formats(integral_constant<int, kMmGelu>{});
+    else formats(integral_constant<int, kMmPlain>{});
+}
+}  // namespace
+
 hipError_t launch_gemm_kq(MmArgs a, int n_col_tiles, hipStream_t st) {
     // Many input rows: k_gemm_wide, the image read once per 64 (or 32) rows
     // instead of once per 16.  It needs enough tiles: k_gemm_kq's waves split
@@ -2463,13 +2498,13 @@ hipError_t launch_gemm_kq(MmArgs a, int n_col_tiles, hipStream_t st) {
     const size_t lds = fq ? fused_lds_bytes(16, a.n_in, a.norm_w != nullptr) : 0;
     const dim3 g((unsigned)tiles, (unsigned)n_col_tiles);
     if (tiles < 128) {
-        if (fq) k_gemm_kq<16, 1, true><<<g, 1024, lds, st>>>(a);
-        else k_gemm_kq<16, 1, false><<<g, 1024, 0, st>>>(a);
+        if (fq) launch_kq<16, 1, true>(a, g, lds, st);
+        else launch_kq<16, 1, false>(a, g, 0, st);
     } else if (n_col_tiles == 1) {
-        if (fq) k_gemm_kq<8, 1, true><<<g, 512, lds, st>>>(a);
-        else k_gemm_kq<8, 1, false><<<g, 512, 0, st>>>(a);
+        if (fq) launch_kq<8, 1, true>(a, g, lds, st);
+        else launch_kq<8, 1, false>(a, g, 0, st);
     } else {
-        k_gemm_kq<8, 2, false><<<dim3((unsigned)tiles, (unsigned)((n_col_tiles + 1) / 2)), 512, 0, st>>>(a);
+        launch_kq<8, 2, false>(a, dim3((unsigned)tiles, (unsigned)((n_col_tiles + 1) / 2)), 0, st);
     }
     return hipGetLastError();
 }
