@@ -258,8 +258,8 @@ def test_q8_0_products_with_norm_bias_and_biases(P):
     """A Q8_0 file's encoder Q/K/V (all three Q8_0, src/voxtral-quantize.cpp:
     95-96): the q8_0 image of every row (codes in the products' lane order,
     the fp16 d of every 32-element block in the sums' place) is ggml's x86
-    quantize_row_q8_0 of the normed row bit for bit, through the fused (P <= 4)
-    and the separate quantization alike; the outputs are within the bound."""
+    quantize_row_q8_0 of the normed row bit for bit, through the fused (few
+    rows) and the separate quantization alike; the outputs are within the bound."""
     rng = np.random.default_rng(8000 + P)
     n_in = 1280
     mats = [(vkv.Q8_0, 1280, True), (vkv.Q8_0, 1280, False), (vkv.Q8_0, 1280, True)]
@@ -350,20 +350,23 @@ def test_q8_0_matches_the_single_row_kernel_and_rejects_mixing():
                    ws_ptr, ws_b, hip_stream=stream_ptr())
 
 
-@pytest.mark.parametrize("P", [3, 11, 24])   # quantized inside; one column tile; two
+# quantized inside (up to 6 rows of K-quants, 8 of Q8_0), and by a launch of
+# its own; one column tile, two
+@pytest.mark.parametrize("P", [3, 6, 7, 8, 9, 16, 24])
 @pytest.mark.parametrize("n_in,n_rows", [(1280, 500), (1280, 2100), (3072, 2063)])   # 16 and 8 waves
 @pytest.mark.parametrize("norm", [False, True])
 def test_a_matrix_gives_the_same_rows_in_every_kind_of_call(P, n_in, n_rows, norm):
     """Calls of one format and of both K-quants, and each epilogue, run kernels
-    of their own: a matrix's rows are the same bits alone and beside another
-    format's; SwiGLU (its waves split K in halves: the f32 order of the sums,
+    of their own: a matrix's rows are the same bits alone, beside another
+    format's and in a call of more rows; SwiGLU (its waves split K in halves: the f32 order of the sums,
     1e-5 x sum |w||x|) and GELU are the functions of the plain products."""
     rng = np.random.default_rng(P + n_in + n_rows + norm)
-    x = torch.from_numpy(rng.standard_normal((P, n_in)).astype(np.float32)).to(dev()) * 0.5
+    rows = torch.from_numpy(rng.standard_normal((24, n_in)).astype(np.float32)).to(dev()) * 0.5
+    x = rows[:P]
     nw = torch.from_numpy(rng.uniform(0.5, 1.5, n_in).astype(np.float32)).to(dev())
-    t, wp, wb = workspace(P, n_in)
+    t, wp, wb = workspace(24, n_in)
 
-    def call(mats, epilogue=vkv.MV_STORE):
+    def call(mats, epilogue=vkv.MV_STORE, P=P):
         ys = [torch.full((P, n_rows), np.nan, device=dev()) for _ in mats]
         vkv.matmul(x.data_ptr(), P, n_in, [(w.data_ptr(), dt, n_rows, y.data_ptr()) for (dt, w), y in zip(mats, ys)],
                    wp, wb, norm_w_ptr=nw.data_ptr() if norm else None, eps=EPS, epilogue=epilogue,
@@ -376,6 +379,8 @@ def test_a_matrix_gives_the_same_rows_in_every_kind_of_call(P, n_in, n_rows, nor
     for mix in ([vkv.Q4_K, vkv.Q6_K], [vkv.Q6_K, vkv.Q4_K], [vkv.Q8_0, vkv.Q8_0]):
         for dt, y in zip(mix, call([(dt, w[dt][0]) for dt in mix])):
             assert torch.equal(y, alone[dt][0])
+    for dt in types:
+        assert torch.equal(call([(dt, w[dt][0])], P=24)[0][:P], alone[dt][0])
     h = x * torch.rsqrt((x * x).mean(1, keepdim=True) + EPS) * nw if norm else x
     for dt in types:
         g, u = (y.double() for y in alone[dt])

@@ -2510,21 +2510,21 @@ hipError_t launch_gemm_kq(MmArgs a, int n_col_tiles, hipStream_t st) {
 }
 
 // Whether the call's input image is quantized inside its work groups: at most
-// kFqRows input rows (the realtime encoder's 4-frame chunks, single adapter
-// groups), every 16-lane group with at most kFqRounds (row, block) tasks, and
-// the image in LDS beside the product's own.  Measured on MI355X against the
-// separate k_q8k_rows launch, with 16-row tiles T of K inputs: 4 rows T = 80,
-// K = 5120 10.4 against 11.7 us, T = 192, K = 4096 8.6 against 9.8, T = 384,
-// K = 1280 9.4 against 9.0; 8 rows 9.1 against 8.3 (T = 80, K = 2048) and
-// 11.2 against 9.1 (T = 384, K = 1280); 16 rows 12.4 against 8.9 (T = 80, K =
-// 2048), and with several column tiles every one of them quantized again.
-constexpr int kFqRows = 4;
+// kFqRows input rows (kFqRowsQ80 of Q8_0's, a cheaper quantization), every
+// 16-lane group with at most kFqRounds (row, block) tasks, and the image in LDS
+// beside the product's own.  Each work group repeats the quantization, where
+// k_q8k_rows is one more dependent launch.  Measured on MI355X, whole encoder
+// chunks (inside against separate, ms): K-quants 4 frames 1.54 / 1.67, 5
+// 1.63 / 1.70, 6 1.69 / 1.71, 8 1.81 / 1.75, 12 1.94 / 1.79; Q8_0 4 frames
+// 1.60 / 1.87, 5 1.65 / 1.88, 6 1.69 / 1.89, 8 1.85 / 1.94, 12 2.00 / 1.98.
+constexpr int kFqRows = 6, kFqRowsQ80 = 8;
 bool gemm_fused_ok(const MmArgs &a) {
     int tiles = 0;
     for (int k = 0; k < a.n_outs; ++k)
         if (!(a.swiglu && k == 1)) tiles += (a.out[k].n_rows + 15) / 16;
     const int waves = tiles < 128 ? 16 : 8;
-    return a.n_cols <= kFqRows && a.n_cols * (a.n_in / 256) <= kFqRounds * 4 * waves &&
+    const int rows = a.out[0].dtype == VKV_DTYPE_Q8_0 ? kFqRowsQ80 : kFqRows;
+    return a.n_cols <= rows && a.n_cols * (a.n_in / 256) <= kFqRounds * 4 * waves &&
            (!a.norm_w || a.n_in <= kFqNormPer * 64 * waves) &&
            fused_lds_bytes(16, a.n_in, a.norm_w != nullptr) <= 128 * 1024;
 }
