@@ -288,12 +288,15 @@ def test_prompt_two_layers(cap, P, N, acap, kind):
     del keep, arr, at
 
 
-def test_prompt_longer_than_one_embedding_launch():
-    """300 tokens (two embedding launches), no audio: the same bits as the
-    composed sequence."""
-    rng = np.random.default_rng(300)
-    n_layers, vocab, cap, N = 1, 2048, 512, 300
-    m = tok.make_model(rng, n_layers, vocab)
+@pytest.mark.parametrize("N,kind", [(64, "q4km"), (130, "q4km"), (300, "q4km"), (64, "q8_0"),
+                                    (130, "q8_0"), (300, "q8_0")])
+def test_long_prompts(N, kind):
+    """Prompts in the many-row products (the Q/K/V call with its RoPE, of both
+    K-quants or of Q8_0, in each of their tile shapes), 300 tokens in two
+    embedding launches, no audio: the same bits as the composed sequence."""
+    rng = np.random.default_rng(N)
+    n_layers, vocab, cap = 1, 2048, 512
+    m = tok.make_model(rng, n_layers, vocab, kind)
     model, keep, arr = tok.upload_model(m)
     tokens = [int(t) for t in rng.integers(0, vocab, N)]
     sp = stream_ptr()

@@ -2406,13 +2406,68 @@ hipError_t launch_gemm_wide(MmArgs a, hipStream_t st) {
     const dim3 g((unsigned)tiles, (unsigned)((a.n_cols + 16 * CT - 1) / (16 * CT)));
     const bool q80 = a.out[0].dtype == VKV_DTYPE_Q8_0;
     constexpr int NT = 64 * RT * (SW ? 2 : 1);
-    if (q80) k_gemm_wide<CT, RT, SW, true><<<g, NT, 0, st>>>(a);
-    else k_gemm_wide<CT, RT, SW, false><<<g, NT, 0, st>>>(a);
+    // (no 2x4 form for Q8_0: nowhere measured the best one by more than 3%)
+    if constexpr (CT == 2 && RT == 4) {
+        if (q80) return hipErrorInvalidValue;
+    } else if (q80) {
+        k_gemm_wide<CT, RT, SW, true><<<g, NT, 0, st>>>(a);
+        return hipGetLastError();
+    }
+    k_gemm_wide<CT, RT, SW, false><<<g, NT, 0, st>>>(a);
     return hipGetLastError();
 }
 }  // namespace
 
 namespace {
+// Which k_gemm_wide (16-input column tiles x 16-row tiles per work group), if
+// any, a call of several 16-input tiles takes instead of k_gemm_kq, whose waves
+// split K and so fill the chip with fewer tiles.  T 16-row tiles, P inputs; the
+// work groups of each form are counted against the chip's 256 CUs, which run
+// four of two waves at once.  Measured on MI355X, products of T = 80 .. 768
+// tiles and SwiGLU pairs of 40 .. 576 at 20 input counts from 17 to 503, cold
+// weights, quantization launch included (us, k_gemm_kq and the forms):
+//   K-quants    T = 80, K = 2048    96: 12.2, 2x2 14.0   128: 15.3, 14.2
+//               T = 80, K = 5120   128: 26.0, 2x2 26.8   160: 32.2, 26.9
+//               T = 192, K = 4096   64: 21.4, 2x2 21.1   96: 28.7, 2x4 21.3 (2x2 25.1)
+//               T = 192, K = 9216   80: 44.3, 2x4 49.6   96: 50.3, 49.8   320: 117, 4x4 71.5 (2x2 82.3)
+//               T = 384, K = 3072   38: 18.9, 2x2 21.1   49: 22.7, 21.3   160: 42.9, 27.3 (4x4 33.4)
+//                                  192: 48.8, 4x4 34.4 (2x2 31.4)   503: 114, 44.8 (2x2 62.7)
+//     SwiGLU    T = 320, K = 1280   20: 13.2, 2x2 11.9   128: 26.1, 16.4 (4x2 18.1)
+//               T = 576, K = 3072   32: 33.4, 2x2 23.4   97: 71.9, 4x2 39.3 (2x2 41.3)   503: 299, 103
+//   Q8_0        T = 80, K = 2048    96: 15.0, 2x2 16.2   128: 19.7, 16.4
+//               T = 192, K = 4096  128: 33.0, 2x2 36.1   160: 42.0, 38.0   320: 77, 4x4 52 (2x2 69)
+//               T = 384, K = 3072   65: 31.5, 2x2 33.2   96: 35.0, 33.8   129: 45.8, 42.3 (4x4 48.9)
+//     SwiGLU    T = 320, K = 1280   64: 20.5, 2x2 20.7   80: 22.3, 21.2   97: 27.8, 4x2 24.0 (2x2 26.9)
+//               T = 576, K = 3072   38: 50.8, 4x2 53.5   49: 58.0, 54.8   503: 367, 192
+enum class WideForm { kNone, k2x2, k2x4, k4x2, k4x4 };
+WideForm wide_form(const MmArgs &a) {
+    if (a.x || a.n_cols <= 16) return WideForm::kNone;
+    int64_t t = 0;
+    for (int k = 0; k < a.n_outs; ++k)
+        if (!(a.swiglu && k == 1)) t += (a.out[k].n_rows + 15) / 16;
+    const bool q80 = a.out[0].dtype == VKV_DTYPE_Q8_0, q4 = a.out[0].dtype == VKV_DTYPE_Q4_K;
+    const int64_t p = a.n_cols, c32 = (p + 31) / 32, c64 = (p + 63) / 64;
+    const int64_t g2x2 = (t + 1) / 2 * c32, g2x4 = (t + 3) / 4 * c32;
+    const int64_t g4x2 = (t + 1) / 2 * c64, g4x4 = (t + 3) / 4 * c64;
+    if (a.swiglu) {
+        // 64 inputs from where 32 leave the CUs more than one round of work
+        // groups; sooner for the costlier operands of Q6_K and Q8_0, where 64
+        // make one round
+        const bool four = g2x2 > (q4 ? 640 : 512) || (!q4 && g2x2 > 256 && g4x2 <= 256);
+        if (t * p < (!q80 ? 6144 : four && g4x2 > 256 ? 27648 : 24576)) return WideForm::kNone;
+        return four ? WideForm::k4x2 : WideForm::k2x2;
+    }
+    // Few tiles: k_gemm_kq's 16 waves split K, the better the longer it is.
+    // Q8_0 (a float scale per 32 elements in both kernels) wins later.
+    const bool wide = t < 128 ? t * ((p + 15) / 16) >= (a.n_in > 4096 ? 800 : 560)
+                              : t * p >= (q80 ? 30720 : p >= 96 ? 10240 : 16384);
+    if (!wide) return WideForm::kNone;
+    // 64 x 64 from where 32 x 32 make more than a round of the chip's SIMDs;
+    // 64 rows x 32 inputs where that is one work group per CU at most
+    if (g2x2 > 1024 || (!q4 && g2x2 > 768 && g4x4 <= 256)) return WideForm::k4x4;
+    return !q80 && g2x2 > 256 && g2x4 <= 256 ? WideForm::k2x4 : WideForm::k2x2;
+}
+
 // k_gemm_kq for the call's weight formats and epilogue
 template <int W, int CT, bool FQ>
 void launch_kq(const MmArgs &a, dim3 g, size_t lds, hipStream_t st) {
@@ -2439,38 +2494,13 @@ void launch_kq(const MmArgs &a, dim3 g, size_t lds, hipStream_t st) {
 }  // namespace
 
 hipError_t launch_gemm_kq(MmArgs a, int n_col_tiles, hipStream_t st) {
-    // Many input rows: k_gemm_wide, the image read once per 64 (or 32) rows
-    // instead of once per 16.  It needs enough tiles: k_gemm_kq's waves split
-    // K, so it fills the chip with few.  Measured on MI355X (us, k_gemm_kq
-    // against k_gemm_wide) with T 16-row tiles and P input rows: T = 384,
-    // K = 3072 (Q/K/V): P = 38 19.7 / 21.5, 64 22.6 / 22.2, 128 35.7 / 25.1,
-    // 503 114 / 57; T = 192, K = 4096: 64 22.1 / 20.5, 96 29.6 / 21.2, 503
-    // 97 / 40; T = 192, K = 9216 (Q6_K): 64 38.6 / 40.9, 128 54.1 / 50.7, 503
-    // 180 / 95; T = 80, K = 2048: 64 12.5 / 13.9, 128 16.7 / 14.3; SwiGLU
-    // with T = 576: 20 30.3 / 22-23, 38 37.7 / 30, 503 299 / 119, T = 320:
-    // 20 13.7 / 12, 128 28.3 / 18.7.
-    if (!a.x && n_col_tiles > 1) {
-        int t16 = 0;
-        for (int k = 0; k < a.n_outs; ++k)
-            if (!(a.swiglu && k == 1)) t16 += (a.out[k].n_rows + 15) / 16;
-        const int64_t work = (int64_t)t16 * a.n_cols;
-        // (Q8_0, a float scale per 32 elements in both: from more tiles on;
-        // T = 576, SwiGLU: 38 51.6 / 62.6, 61 61.0 / 58.0, 503 368 / 206;
-        // T = 192: 128 33.4 / 38.5, 251 59.9 / 54.8)
-        const bool q80 = a.out[0].dtype == VKV_DTYPE_Q8_0;
-        if (a.swiglu) {
-            // two waves' rows x 64 inputs from 512 tiles of 16 x 64, else x 32
-            if (work >= 32768) return launch_gemm_wide<4, 2, true>(a, st);
-            if (work >= (q80 ? 24576 : 6144)) return launch_gemm_wide<2, 2, true>(a, st);
-        } else if (work >= (q80 ? 32768 : a.n_cols >= 96 ? 10240 : 16384)) {
-            // 64 inputs per work group while that leaves every SIMD a wave,
-            // else 32; then work groups of 4 waves where they are no more
-            // than the CUs, of 2 where those would leave CUs idle or double up
-            const int64_t w32 = (int64_t)t16 * ((a.n_cols + 31) / 32);
-            if ((int64_t)t16 * ((a.n_cols + 63) / 64) >= 1024) return launch_gemm_wide<4, 4, false>(a, st);
-            if (w32 > 512 && w32 <= 1024) return launch_gemm_wide<2, 4, false>(a, st);
-            return launch_gemm_wide<2, 2, false>(a, st);
-        }
+    switch (wide_form(a)) {
+    case WideForm::k2x2:
+        return a.swiglu ? launch_gemm_wide<2, 2, true>(a, st) : launch_gemm_wide<2, 2, false>(a, st);
+    case WideForm::k2x4: return launch_gemm_wide<2, 4, false>(a, st);
+    case WideForm::k4x2: return launch_gemm_wide<4, 2, true>(a, st);
+    case WideForm::k4x4: return launch_gemm_wide<4, 4, false>(a, st);
+    case WideForm::kNone: break;
     }
     // the 16-row tiles of each matrix are consecutive work groups
     int tiles = 0;
@@ -2493,7 +2523,7 @@ hipError_t launch_gemm_kq(MmArgs a, int n_col_tiles, hipStream_t st) {
     // tiles (32 input rows) per work group at most: a third set of
     // accumulators spills at four waves per SIMD, and measured slower.
     // A fused-input call (a.x) quantizes each work group's input rows into
-    // dynamic LDS (the caller checked gemm_fused_lds).
+    // dynamic LDS (gemm_fused_ok bounds its size).
     const bool fq = a.x != nullptr;   // (one column tile)
     const size_t lds = fq ? fused_lds_bytes(16, a.n_in, a.norm_w != nullptr) : 0;
     const dim3 g((unsigned)tiles, (unsigned)n_col_tiles);
