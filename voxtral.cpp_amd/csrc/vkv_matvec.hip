@@ -1702,6 +1702,10 @@ __device__ __forceinline__ void gemm_body(const MmArgs &a, const MmOut &o0, cons
 // epilogues in each and it took 1.667 or 1.699 ms on a Q8_0 file as they moved,
 // 1.59 on a K-quant one; with their own, 47 KB (Q8_0), it takes 1.60 and 1.52.
 //
+// Four waves per SIMD at most: Q8_0's SwiGLU instance alone has registers for
+// six, and with three work groups on a CU instead of two a 9216-row pair of 12
+// inputs took 31.3 us against 30.1.
+//
 // (the body is in the kernel itself: a reference to the by-value kernel
 // argument passed through one more inlined function made the compiler copy
 // the argument to scratch memory)
@@ -1715,7 +1719,7 @@ __host__ __device__ constexpr size_t fused_lds_bytes(int cols, int n_in, bool no
 }
 
 template <int W, int CT, bool FQ, int FMT, int EPI>
-__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) k_gemm_kq(MmArgs a) {
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4, 4))) k_gemm_kq(MmArgs a) {
     __shared__ uint32_t hdr[W][16][6];
     __shared__ float red[CT][W][16][17];
     int seg = 0;
