@@ -1696,19 +1696,6 @@ __device__ __forceinline__ void gemm_body(const MmArgs &a, const MmOut &o0, cons
     }
 }
 
-// FMT, EPI: the call's weight formats (kWK: both K-quants) and epilogue, each
-// kernel with only those, for the instruction cache (see k_matvec).  The
-// 4-frame encoder chunk's kernels were 102 KB with all three formats and
-// epilogues in each and it took 1.667 or 1.699 ms on a Q8_0 file as they moved,
-// 1.59 on a K-quant one; with their own, 47 KB (Q8_0), it takes 1.60 and 1.52.
-//
-// Four waves per SIMD at most: Q8_0's SwiGLU instance alone has registers for
-// six, and with three work groups on a CU instead of two a 9216-row pair of 12
-// inputs took 31.3 us against 30.1.
-//
-// (the body is in the kernel itself: a reference to the by-value kernel
-// argument passed through one more inlined function made the compiler copy
-// the argument to scratch memory)
 // Fused input image in dynamic LDS: codes, block scales, 32-element sums,
 // per-task sums of squares (the norm's first pass).
 __host__ __device__ constexpr size_t al16(size_t b) { return (b + 15) & ~(size_t)15; }
@@ -1718,8 +1705,22 @@ __host__ __device__ constexpr size_t fused_lds_bytes(int cols, int n_in, bool no
            (norm ? (size_t)3 * n_in * 4 : 0);
 }
 
+// FMT, EPI: the call's weight formats (kWK: both K-quants) and epilogue, each
+// kernel with only those, for the instruction cache (see k_matvec).  The
+// 4-frame encoder chunk's kernels were 102 KB with all three formats and
+// epilogues in each and it took 1.667 or 1.699 ms on a Q8_0 file as they moved,
+// 1.59 on a K-quant one; with their own, 47 KB (Q8_0), it takes 1.60 and 1.52.
+//
+// With one column tile, four waves per SIMD at most: Q8_0's SwiGLU instance
+// alone has registers for six, and with three work groups on a CU instead of
+// two a 9216-row pair of 12 inputs took 31.3 us against 30.1.
+//
+// (the body is in the kernel itself: a reference to the by-value kernel
+// argument passed through one more inlined function made the compiler copy
+// the argument to scratch memory)
 template <int W, int CT, bool FQ, int FMT, int EPI>
-__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4, 4))) k_gemm_kq(MmArgs a) {
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4, CT == 1 ? 4 : 8)))
+k_gemm_kq(MmArgs a) {
     __shared__ uint32_t hdr[W][16][6];
     __shared__ float red[CT][W][16][17];
     int seg = 0;
