@@ -94,3 +94,39 @@ def test_rows_beyond_the_format_stay_with_the_queries_that_see_them(bad):
     a, b = both(128, 8, 32, 1, 64, call)
     assert np.isfinite(b[0, :at]).all() and np.array_equal(np.isfinite(a), np.isfinite(b))
     assert np.abs(a[0, :at] - b[0, :at]).max() <= 5e-6 * np.abs(b[0, :at]).max()
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan"), 3e38])
+@pytest.mark.parametrize("win,at", [(12, 17), (1, 16), (40, 0)])
+def test_a_key_beyond_the_format_stays_with_the_queries_that_see_it(bad, win, at):
+    """a K row whose scale overflows f16: the queries that mask it are as
+    without it, those that see it (alone in its 16-key block or in the whole
+    window too) are NaN, not zeros; in the unsplit and the split tile"""
+    n = 40
+    q, k, v = (rows(i, 1, n, w) for i, w in ((3, 4096), (4, 1024), (5, 1024)))
+    k[0, at] = bad
+
+    def prefill(c):
+        out = torch.zeros(1, n, 4096, device=dev())
+        c.decoder_prefill(0, vkv.new_ring(96), 0, 1, n, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+                          128 ** -0.5, hip_stream=stream_ptr())
+        return out
+
+    def window(width):
+        def call(c):
+            out = torch.zeros(1, n, width, device=dev())
+            c.enc_step(0, vkv.enc_plan(0, n, 96, win), win, 0, 1, q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                       out.data_ptr(), 128 ** -0.5, hip_stream=stream_ptr())
+            return out
+        return call
+
+    for shape, call, sees in (((128, 8, 32), prefill, range(at, n)),
+                              ((128, 8, 32), window(4096), range(at, min(n, at + win))),
+                              ((64, 16, 16), window(1024), range(at, min(n, at + win)))):
+        a, b = both(*shape, 1, 96, call)
+        clean = [i for i in range(n) if i not in sees]
+        assert np.isfinite(b[0, clean]).all() and np.array_equal(np.isfinite(a), np.isfinite(b))
+        if bad == bad:   # (a NaN row is stored as zeros: its largest magnitude is 0)
+            assert np.isnan(a[0, list(sees)]).all()
+        if clean:
+            assert np.abs(a[0, clean] - b[0, clean]).max() <= 5e-6 * np.abs(b[0, clean]).max()

@@ -1873,15 +1873,16 @@ typedef float float4_t __attribute__((ext_vector_type(4)));
 // group s runs virtual waves [sW, sW + W); it writes its merged (O, M, L)
 // as a partial, which k_window_merge combines in split order.  Only for
 // GQA 1 (a partial per (query row, head, split)).
-// O / L of N dims to an output row (outputs are 16-byte aligned).
+// O / L of N dims to an output row (outputs are 16-byte aligned): zeros where
+// the row saw no key (L = 0), NaN where a score it saw was none (L is NaN).
 template <int N>
 __device__ __forceinline__ void window_store_out(float *p, const float (&o)[N], float l) {
     if constexpr (N == 4) {
         float4 v = make_float4(0, 0, 0, 0);
-        if (l > 0.0f) v = make_float4(o[0] / l, o[1] / l, o[2] / l, o[3] / l);
+        if (l != 0.0f) v = make_float4(o[0] / l, o[1] / l, o[2] / l, o[3] / l);
         *reinterpret_cast<float4 *>(p) = v;
     } else {
-        *p = l > 0.0f ? o[0] / l : 0.0f;
+        *p = l != 0.0f ? o[0] / l : 0.0f;
     }
 }
 
@@ -1911,6 +1912,10 @@ __device__ __forceinline__ void window_merge_waves(const WindowArgs &a, const fl
             for (int e = 0; e < N; ++e) O[e] = fmaf(o[e], f, O[e]);
             L = fmaf(sm_l[w][r], f, L);
         }
+    } else {
+        // no key seen, or none with a score: the sums are 0 or NaN
+#pragma unroll
+        for (int w = 0; w < W; ++w) L += sm_l[w][r];
     }
     if constexpr (SPL > 1) {
         static_assert(N == 4, "whole float4s");
@@ -2194,6 +2199,9 @@ __global__ void __launch_bounds__(256) k_window_merge(const float *part_o, const
             O[3] = fmaf(o[s].w, f, O[3]);
             L = fmaf(l[s], f, L);
         }
+    } else {
+#pragma unroll
+        for (int s = 0; s < SPL; ++s) L += l[s];
     }
     window_store_out<4>(out + v * D + d, O, L);
 }
