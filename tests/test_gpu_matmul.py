@@ -397,3 +397,25 @@ def test_a_matrix_gives_the_same_rows_in_every_kind_of_call(P, n_in, n_rows, nor
         sg = g / (1 + torch.exp(-g))
         bound = REL * (1.1 * mags[0] * u.abs() + sg.abs() * mags[1]) + 1e-6 * (sg * u).abs()
         assert ((y - sg * u).abs() <= bound + 1e-30).all()
+
+
+@pytest.mark.parametrize("dtype", [vkv.Q4_K, vkv.Q6_K, vkv.Q8_0])
+@pytest.mark.parametrize("P", [3, 12, 24, 160])   # quantized inside, one and two column tiles, the wide kernel
+def test_weights_aligned_to_four_bytes(dtype, P):
+    """weights are promised 4-byte alignment only: the same bits at every such
+    offset as at a 256-byte aligned address"""
+    rng = np.random.default_rng(P)
+    n_in, n_rows = 1280, 2100
+    w = to_dev(random_matrix(rng, dtype, n_rows, n_in, 0.05))
+    x = to_dev(rng.standard_normal((P, n_in)).astype(np.float32))
+    t, wp, wb = workspace(P, n_in)
+    want = None
+    for off in (0, 4, 8, 12):
+        moved = torch.zeros(w.numel() + 256, dtype=torch.uint8, device=dev())
+        moved[off:off + w.numel()] = w
+        y = torch.full((P, n_rows), np.nan, device=dev())
+        vkv.matmul(x.data_ptr(), P, n_in, [(moved.data_ptr() + off, dtype, n_rows, y.data_ptr())], wp, wb,
+                   hip_stream=stream_ptr())
+        torch.cuda.synchronize()
+        want = y if off == 0 else want
+        assert torch.isfinite(y).all() and torch.equal(y, want), off

@@ -1632,9 +1632,15 @@ __device__ __forceinline__ void gemm_body(const MmArgs &a, const MmOut &o0, cons
                                  : (o0.add ? o0.add : o0.y);
     const int64_t e2i = swiglu ? ot_row : o0.rope ? min(row0 + (ot_r ^ 1), o0.n_rows - 1) : ot_at;
     const float e_2 = e2p[e2i];
-    // the angle's pair (no RoPE: the weights' first bytes, unused)
-    const float2 e_cs = *(o0.rope ? a.rope_tab + (int64_t)ot_col * (a.rope_hd >> 1) + ((ot_row % a.rope_hd) >> 1)
-                                  : reinterpret_cast<const float2 *>(o0.w));
+    // the angle's pair (no RoPE: the weights' first bytes, unused; they are
+    // 4-byte aligned, no more)
+    struct __attribute__((packed, aligned(4))) Pair4 {
+        float c, s;
+    };
+    const Pair4 e_p = *(o0.rope ? reinterpret_cast<const Pair4 *>(a.rope_tab + (int64_t)ot_col * (a.rope_hd >> 1) +
+                                                                  ((ot_row % a.rope_hd) >> 1))
+                                : reinterpret_cast<const Pair4 *>(o0.w));
+    const float2 e_cs = make_float2(e_p.c, e_p.s);
     // the wave's blocks b, b + kw, b + 2 kw, ...: one block's fragments at a
     // time (occupancy, not a second register set, covers the load latency);
     // the first block's (w_first) were requested by the caller
