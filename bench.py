@@ -1741,8 +1741,8 @@ def main():
                               "residual) + final norm; dim 1280, 32 heads x 64, hidden 5120",
                   "layers": E_LAYERS, "window": E_WIN, "frames_per_chunk": E_CHUNK,
                   "bytes_per_chunk": bytes_step, "keys_per_query_block": n_keys}
-        kernel = ("conv stem (k_im2col_f16 + k_gemm_f16, x2) + 32 x (k_q8k_rows + k_gemm_kq, x4; "
-                  "k_rope; k_window_mfma) + final norm")
+        kernel = ("conv stem (k_im2col_f16 + k_gemm_f16, x2) + k_rope_pairs + 32 x (k_q8k_rows + "
+                  "k_gemm_kq, x4; k_window_mfma_f32_64_split + k_window_merge) + final norm")
     elif args.workload in ("adapter_q4km", "adapter_group_q4km"):
         ng = wl["groups"]
         total_ms, step_ms, wall = gpu_adapter(ng, args.steps, args.warmup)
@@ -1802,7 +1802,7 @@ def main():
                               "SwiGLU, W2 + residual), final norm, 131072-row logits, argmax",
                   "layers": LAYERS, "dim": DIM, "hidden": HIDDEN, "vocab": VOCAB,
                   "prompt_tokens": P_TOKENS, "bytes_per_prompt": bytes_step}
-        kernel = "whole prompt (k_gemm_kq, k_q8k_rows, k_window_mfma, k_matvec launches)"
+        kernel = "whole prompt (k_gemm_kq, k_gemm_wide, k_q8k_rows, k_window_mfma, k_matvec launches)"
     elif args.workload in ("decoder_token_q4km", "decoder_token_q8_0"):
         total_ms, step_ms, wall = gpu_token(args.steps, args.warmup)
         bytes_step = token_bytes()

@@ -1553,7 +1553,7 @@ __device__ __forceinline__ void gemm_dot(const GFragQ6 &f, const GFragX &x, cons
 // vkv_rope's arithmetic: the angle pos * ts^pair by the running f32 product,
 // cos/sin in double rounded to f32.  Evaluated once for all layers of a prompt
 // or an encoder chunk: in every layer's products the double evaluation was
-// ~4 us of a 38-token Q/K/V call's 19 and spilled k_gemm_wide's registers.
+// ~4 us of a 38-token Q/K/V call's 19, and more registers in k_gemm_wide.
 __global__ void __launch_bounds__(256) k_rope_pairs(float2 *tab, int n, int pairs, int64_t pos0, float ts) {
 #pragma clang fp contract(off)
     const int i = (int)blockIdx.x * 256 + (int)threadIdx.x;
@@ -1807,14 +1807,16 @@ k_gemm_kq(MmArgs a) {
 // ---------------------------------------------------------------------------
 // The same products for many input rows.  k_gemm_kq gives each 16-row tile its
 // own work group, which reads the whole input image again: at 503 input rows
-// Q/K/V (6144 x 3072) took 114 us, W1/W3 298 us, an eighth of the int8 rate's
-// share.  Here a work group owns 16 RT weight rows x 16 CT input rows: wave w
-// rows [16 w, 16 w + 16), every wave the same input columns, whose image block
-// is staged in LDS once per K block (double-buffered, one barrier per block).
-// The same calls take 47 and 107 us; bound by the ~5 VALU operations that an
-// output takes per block and those that make the operands (VALU ~5 clocks an
-// operation beside 16 for a product, measured), then by the few waves that
-// 3072-row matrices leave (one or two per SIMD).
+// Q/K/V (6144 x 3072) took 114 us, W1/W3 301.  Here a work group owns 16 RT
+// weight rows x 16 CT input rows: wave w rows [16 w, 16 w + 16), every wave the
+// same input columns, whose image block is staged in LDS once per K block
+// (double-buffered, one barrier per block).  The same calls take 46 and 104 us
+// (quantization launch included), bound by vector issue: 9.5 (Q4_K) and 11.4
+// (Q6_K) vector instructions per MFMA, a half (Q4_K) or a quarter (Q6_K) of them
+// the outputs' block terms, the rest the operands, made again for every 16 CT
+// inputs.  W1/W3 issue 37 k of them per SIMD, 62 us of the 104 at 4 clocks
+// each.  Narrow matrices leave it too few waves (80 tiles x 128 inputs: 320 on
+// 1024 SIMDs, each a serial chain over K).
 //
 // Products per 256-block.  The 6-bit scales are folded into the int8 operand
 // instead of multiplying each 32-element sum on the VALU, which took ~70 of
@@ -2066,9 +2068,11 @@ struct WideOps<kWQ8> {
 constexpr int kWideCol = 272;   // bytes per staged column: 256 codes, padded against bank conflicts
 
 // Blocks requested ahead: two where the launch rule leaves a SIMD one wave
-// (4 waves x 32 inputs; K = 9216, 128 inputs: 49.8 us against 55.3), else one,
+// (4 waves x 32 inputs; K = 9216, 128 inputs: 50.5 us against 56.0), else one,
 // whose registers leave room for a third wave per SIMD (503 inputs, K = 3072:
-// 47.9 us against 57.4 for Q/K/V, 111 against 121 for W1/W3).
+// 45.7 us against 54.8 for Q/K/V, 104 against 114 for W1/W3).  At three waves
+// the 64 x 64 form still spills: 10 of Q8_0's registers, three inside the block
+// loop; 16 of the K-quants', outside it.
 __host__ __device__ constexpr int wide_pre(int ct, int rt) { return ct == 2 && rt == 4 ? 2 : 1; }
 
 // Two image blocks and the waves' block headers
